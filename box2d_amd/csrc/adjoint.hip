@@ -837,7 +837,7 @@ __global__ __launch_bounds__( kAdjointThreads ) void AdjointKernel( const Adjoin
 
 	const int ncMax = W.ncMax;
 	ConstraintSoA c;
-	c.f = FieldTable{ W.cfields, ncMax };
+	c.f = RowTable{ W.cfields, ncMax };
 	c.bodyA = W.cints;
 	c.bodyB = W.cints + ncMax;
 	c.contactId = W.cints + 2 * ncMax;
@@ -1040,6 +1040,7 @@ __global__ __launch_bounds__( kAdjointThreads ) void AdjointKernel( const Adjoin
 		__syncthreads();
 
 		const int colors = hdr.activeColorCount;
+		auto noRolling = []( const ContactRow& ) { return false; };
 		auto opTape = [&]( int sub, int stage ) { return W.opTape + (size_t)( ( sub * 3 + stage ) * kOpFieldCount ) * ncMax; };
 		float* posTape = W.opTape + (size_t)W.subStepMax * 3 * kOpFieldCount * ncMax;
 		auto record = [&]( float* t, int i ) {
@@ -1102,7 +1103,7 @@ __global__ __launch_bounds__( kAdjointThreads ) void AdjointKernel( const Adjoin
 						}
 						else
 						{
-							SolveContact( c, i, B, true, p.inv_h, contactSpeed, false );
+							SolveContact<true>( c, i, B, p.inv_h, contactSpeed, noRolling );
 						}
 					}
 					__syncthreads();
@@ -1141,7 +1142,7 @@ __global__ __launch_bounds__( kAdjointThreads ) void AdjointKernel( const Adjoin
 					{
 						int i = start + q;
 						record( t, i );
-						SolveContact( c, i, B, false, p.inv_h, contactSpeed, false );
+						SolveContact<false>( c, i, B, p.inv_h, contactSpeed, noRolling );
 					}
 					__syncthreads();
 				}
@@ -1908,10 +1909,10 @@ int b2amd_Tape_Backward( b2amd_Tape* tape, const b2amd_BodyState* finalGrad, b2a
 		a.sims = t->sims[i];
 		float* base = scratch + scratchOff[k];
 		size_t nc = (size_t)ncMax[k];
+		a.cfields = base; // first: its rows are read as float4
+		base += (size_t)kcFieldCount * nc;
 		a.opTape = base;
 		base += (size_t)subMax[k] * 3 * kOpFieldCount * nc + (size_t)subMax[k] * 3 * nbMax[k];
-		a.cfields = base;
-		base += (size_t)kcFieldCount * nc;
 		a.cints = reinterpret_cast<int*>( base );
 		base += 6 * nc;
 		a.cadj = base;

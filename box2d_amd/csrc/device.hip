@@ -452,16 +452,6 @@ B2G_DEV void PrepareContactsBody( const PrepareArgs& a, int i )
 	b2Vec2 vB = a.states[bodyIdB].linearVelocity;
 	float wB = a.states[bodyIdB].angularVelocity;
 
-	c.f[kcInvMassA][i] = mA;
-	c.f[kcInvMassB][i] = mB;
-	c.f[kcInvIA][i] = iA;
-	c.f[kcInvIB][i] = iB;
-
-	{
-		float k = iA + iB;
-		c.f[kcRollingMass][i] = k > 0.0f ? 1.0f / k : 0.0f;
-	}
-
 	Softness soft = a.p.contactSoftness;
 	if ( staticA || staticB )
 	{
@@ -485,64 +475,49 @@ B2G_DEV void PrepareContactsBody( const PrepareArgs& a, int i )
 	float warmStartScale = a.p.enableWarmStarting ? 1.0f : 0.0f;
 
 	b2Vec2 normal = manifold.normal;
-	c.f[kcNormalX][i] = normal.x;
-	c.f[kcNormalY][i] = normal.y;
-	c.f[kcFriction][i] = cs->friction;
-	c.f[kcTangentSpeed][i] = cs->tangentSpeed;
-	c.f[kcRestitution][i] = cs->restitution;
-	c.f[kcRollingResistance][i] = cs->rollingResistance;
-	c.f[kcRollingImpulse][i] = warmStartScale * manifold.rollingImpulse;
-	c.f[kcBiasRate][i] = soft.biasRate;
-	c.f[kcMassScale][i] = soft.massScale;
-	c.f[kcImpulseScale][i] = soft.impulseScale;
+	float k = iA + iB;
+	c.f.Group( kgMass )[i] = make_float4( mA, iA, mB, iB );
+	c.f.Group( kgNormal )[i] = make_float4( normal.x, normal.y, cs->friction, cs->tangentSpeed );
+	c.f.Group( kgSoft )[i] = make_float4( soft.biasRate, soft.massScale, soft.impulseScale, cs->restitution );
+	c.f.Group( kgRolling )[i] =
+		make_float4( cs->rollingResistance, k > 0.0f ? 1.0f / k : 0.0f, warmStartScale * manifold.rollingImpulse, 0.0f );
 
 	b2Vec2 tangent = b2RightPerp( normal );
 
 	for ( int j = 0; j < 2; ++j )
 	{
-		int o = j == 0 ? 0 : ( kcAnchorA2X - kcAnchorA1X );
+		float4 anchor = make_float4( 0.0f, 0.0f, 0.0f, 0.0f );
+		float4 point = anchor;
+		float4 impulse = anchor;
 		if ( j < manifold.pointCount )
 		{
 			const b2ManifoldPoint* mp = manifold.points + j;
 			b2Vec2 rA = mp->anchorA;
 			b2Vec2 rB = mp->anchorB;
-			c.f[kcAnchorA1X + o][i] = rA.x;
-			c.f[kcAnchorA1Y + o][i] = rA.y;
-			c.f[kcAnchorB1X + o][i] = rB.x;
-			c.f[kcAnchorB1Y + o][i] = rB.y;
-			c.f[kcBaseSeparation1 + o][i] = mp->separation - b2Dot( b2Sub( rB, rA ), normal );
-			c.f[kcNormalImpulse1 + o][i] = warmStartScale * mp->normalImpulse;
-			c.f[kcTangentImpulse1 + o][i] = warmStartScale * mp->tangentImpulse;
-			c.f[kcTotalNormalImpulse1 + o][i] = 0.0f;
+			anchor = make_float4( rA.x, rA.y, rB.x, rB.y );
+			impulse.x = warmStartScale * mp->normalImpulse;
+			impulse.y = warmStartScale * mp->tangentImpulse;
+
+			point.x = mp->separation - b2Dot( b2Sub( rB, rA ), normal );
 
 			float rnA = b2Cross( rA, normal );
 			float rnB = b2Cross( rB, normal );
 			float kNormal = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
-			c.f[kcNormalMass1 + o][i] = kNormal > 0.0f ? 1.0f / kNormal : 0.0f;
+			point.y = kNormal > 0.0f ? 1.0f / kNormal : 0.0f;
 
 			float rtA = b2Cross( rA, tangent );
 			float rtB = b2Cross( rB, tangent );
 			float kTangent = mA + mB + iA * rtA * rtA + iB * rtB * rtB;
-			c.f[kcTangentMass1 + o][i] = kTangent > 0.0f ? 1.0f / kTangent : 0.0f;
+			point.z = kTangent > 0.0f ? 1.0f / kTangent : 0.0f;
 
 			b2Vec2 vrA = b2Add( vA, b2CrossSV( wA, rA ) );
 			b2Vec2 vrB = b2Add( vB, b2CrossSV( wB, rB ) );
-			c.f[kcRelativeVelocity1 + o][i] = b2Dot( normal, b2Sub( vrB, vrA ) );
+			point.w = b2Dot( normal, b2Sub( vrB, vrA ) );
 		}
-		else
-		{
-			c.f[kcBaseSeparation1 + o][i] = 0.0f;
-			c.f[kcNormalImpulse1 + o][i] = 0.0f;
-			c.f[kcTangentImpulse1 + o][i] = 0.0f;
-			c.f[kcTotalNormalImpulse1 + o][i] = 0.0f;
-			c.f[kcAnchorA1X + o][i] = 0.0f;
-			c.f[kcAnchorA1Y + o][i] = 0.0f;
-			c.f[kcAnchorB1X + o][i] = 0.0f;
-			c.f[kcAnchorB1Y + o][i] = 0.0f;
-			c.f[kcNormalMass1 + o][i] = 0.0f;
-			c.f[kcTangentMass1 + o][i] = 0.0f;
-			c.f[kcRelativeVelocity1 + o][i] = 0.0f;
-		}
+		const int o = j * ( kgAnchor2 - kgAnchor1 );
+		c.f.Group( kgAnchor1 + o )[i] = anchor;
+		c.f.Group( kgPoint1 + o )[i] = point;
+		c.f.Group( kgImpulse1 + o )[i] = impulse;
 	}
 }
 
@@ -841,14 +816,6 @@ __global__ __launch_bounds__( kWarmBlock ) void IntegrateWarmStartKernel( WarmAr
 	state->angularVelocity = w;
 }
 
-enum ColorStage
-{
-	kStageWarmStart,
-	kStageSolve,
-	kStageRelax,
-	kStageRestitution,
-};
-
 struct ColorArgs
 {
 	ConstraintSoA c;
@@ -877,6 +844,13 @@ B2G_DEV bool GroupAnyNonZero( const ConstraintSoA& c, int f, int colorStart, int
 		}
 	}
 	return false;
+}
+
+// True when the condition holds in any active lane of this lane's aligned group of four.
+B2G_DEV bool LaneGroupAny( bool condition )
+{
+	unsigned long long lanes = __ballot( condition );
+	return ( ( lanes >> ( threadIdx.x & 60 ) ) & 0xF ) != 0;
 }
 
 // Lane t of one graph color of one stage: joints occupy the first jointCount lanes, contacts
@@ -930,12 +904,15 @@ B2G_DEV void ColorLane( const ColorArgs& a, const ColorRange& r, int t, const Bo
 	}
 	else if ( Stage == kStageSolve )
 	{
-		SolveContact( a.c, i, B, true, a.p.inv_h, -a.p.contactSpeed, false );
+		SolveContact<true>( a.c, i, B, a.p.inv_h, -a.p.contactSpeed, []( const ContactRow& ) { return false; } );
 	}
 	else if ( Stage == kStageRelax )
 	{
-		bool rolling = GroupAnyNonZero( a.c, kcRollingResistance, r.contactStart, r.contactCount, k );
-		SolveContact( a.c, i, B, false, a.p.inv_h, -a.p.contactSpeed, rolling );
+		SolveContact<false>( a.c, i, B, a.p.inv_h, -a.p.contactSpeed, [&]( const ContactRow& row ) {
+			// without joints in the color the groups of four are neighbouring lanes
+			return r.jointCount == 0 ? LaneGroupAny( row.rolling.x != 0.0f )
+									 : GroupAnyNonZero( a.c, kcRollingResistance, r.contactStart, r.contactCount, k );
+		} );
 	}
 	else
 	{
@@ -1066,7 +1043,7 @@ static_assert( OverflowLdsBytes() <= 160 * 1024, "overflow chunk must fit in LDS
 template <int Stage>
 __global__ __launch_bounds__( kOverflowThreads ) void OverflowLevelKernel( ColorArgs a, const int* plan )
 {
-	extern __shared__ float lds[];
+	extern __shared__ __align__( 16 ) float lds[];
 	const int C = kOverflowChunkContacts;
 	const int NB = kOverflowChunkBodies;
 	float* fields = lds;
@@ -1077,7 +1054,7 @@ __global__ __launch_bounds__( kOverflowThreads ) void OverflowLevelKernel( Color
 	uint16_t* bflags = reinterpret_cast<uint16_t*>( bf + 7 * NB );
 
 	ConstraintSoA lc = a.c;
-	lc.f = FieldTable{ fields, C };
+	lc.f = RowTable{ fields, C };
 	lc.bodyA = ints;
 	lc.bodyB = ints + C;
 	lc.pointCount = ints + 2 * C;
@@ -1109,11 +1086,11 @@ __global__ __launch_bounds__( kOverflowThreads ) void OverflowLevelKernel( Color
 		int n = c1 - c0;
 		int first = a.contactStart + c0;
 
-		for ( int x = tid; x < kcFieldCount * n; x += kOverflowThreads )
+		for ( int x = tid; x < kcFieldCount / 4 * n; x += kOverflowThreads )
 		{
 			int k = x / n;
 			int j = x - k * n;
-			fields[k * C + j] = a.c.f[k][first + j];
+			lc.f.Group( k )[j] = a.c.f.Group( k )[first + j];
 		}
 		for ( int j = tid; j < n; j += kOverflowThreads )
 		{
@@ -1192,11 +1169,11 @@ __global__ __launch_bounds__( kOverflowThreads ) void OverflowLevelKernel( Color
 			__syncthreads();
 		}
 
-		for ( int x = tid; x < kcFieldCount * n; x += kOverflowThreads )
+		for ( int x = tid; x < kcFieldCount / 4 * n; x += kOverflowThreads )
 		{
 			int k = x / n;
 			int j = x - k * n;
-			a.c.f[k][first + j] = fields[k * C + j];
+			a.c.f.Group( k )[first + j] = lc.f.Group( k )[j];
 		}
 		for ( int j = tid; j < b1 - b0; j += kOverflowThreads )
 		{
@@ -1216,9 +1193,22 @@ __global__ __launch_bounds__( kOverflowThreads ) void OverflowLevelKernel( Color
 //
 // The world's awake body states live in LDS for the duration of the solve (7 floats and 16 flag
 // bits per body, 30 bytes, so kFusedBodyCapacity bodies fit in 160 KB). Colors and stages are
-// separated by workgroup barriers instead of kernel boundaries; constraint fields stream from
-// device memory. Stage order and per-constraint arithmetic are those of the color-kernel path
-// (reference src/solver.c:1090-1170).
+// separated by workgroup barriers instead of kernel boundaries. Stage order and per-constraint
+// arithmetic are those of the color-kernel path (reference src/solver.c:1090-1170).
+//
+// What bounds it is the serial chain of phases (3 stages x colors, plus two, per substep: 116 for a
+// 20-row pyramid), so each phase holds only what depends on the phase before, the velocities' way
+// from LDS through the solve and back. Two lanes share a constraint (PairRow). A color's contacts are
+// cut into chunks of 32 and the chunks of a stage are dealt to the wavefronts in turn, the same way
+// in every stage, so that a wavefront's next chunk is known long before its turn: it loads that
+// chunk's rows as soon as its last one is done, while other wavefronts' colors run, and the barriers
+// between phases wait for LDS only, never for those loads. When no wavefront has more than
+// kResidentRows chunks the rows stay in registers for the whole loop, and the delta-pose part of the
+// solve is computed for all colors at once before the stage's first. Measured per step on an MI355X
+// against one lane per constraint with every field loaded in its phase: 20-row pyramid (590 contacts,
+// 9 colors, resident) 202 -> 48 us; 1000-body mixed pile (about 3000 contacts, 13 colors, streamed)
+// 290 -> 190 us, then bound by its CU's vector instructions; 24x24 net of revolute joints (general)
+// 154 -> 135 us, bound by the joints' scattered loads.
 
 constexpr int kFusedThreads = 1024;
 constexpr int kFusedMaxContacts = 4096;
@@ -1253,37 +1243,12 @@ struct FusedArgs
 	int warmByBody; // 1: warm start body by body, 0: color by color
 };
 
-template <int Stage>
-B2G_DEV void FusedStage( const FusedArgs& a, const LdsBodies& B )
+// Workgroup barrier that orders LDS accesses only: global loads issued before it stay in flight.
+B2G_DEV void LdsBarrier()
 {
-	if ( a.overflowContactCount > 0 || a.overflowJointCount > 0 )
-	{
-		if ( threadIdx.x == 0 )
-		{
-			ColorRange r = { a.overflowJointStart, a.overflowJointCount, a.overflowContactStart, a.overflowContactCount };
-			OverflowSerial<Stage>( a.color, r, B );
-		}
-		__syncthreads();
-	}
-
-	for ( int color = 0; color < a.activeColorCount; ++color )
-	{
-		ColorRange r;
-		r.jointStart = a.colorJointStart[color];
-		r.jointCount = a.colorJointStart[color + 1] - r.jointStart;
-		r.contactStart = a.colorContactStart[color];
-		r.contactCount = a.colorContactStart[color + 1] - r.contactStart;
-		int lanes = r.jointCount + r.contactCount;
-		if ( lanes == 0 || ( Stage == kStageRestitution && r.contactCount == 0 ) )
-		{
-			continue;
-		}
-		for ( int t = threadIdx.x; t < lanes; t += blockDim.x )
-		{
-			ColorLane<Stage>( a.color, r, t, B );
-		}
-		__syncthreads();
-	}
+	__builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup", "local" );
+	__builtin_amdgcn_s_barrier();
+	__builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "workgroup", "local" );
 }
 
 // LDS bytes of a world with `count` awake bodies: slot 0 holds the static identity state, slots
@@ -1294,119 +1259,582 @@ __host__ __device__ inline int FusedLdsBytes( int count )
 	return ( 7 * 4 * cap + 2 * cap + 15 ) & ~15;
 }
 
-// The whole substep loop of one world by the calling workgroup (any block size), body states in
-// the dynamic LDS at lds.
+// A wavefront takes 32 constraints at a time, two lanes each (PairRow).
+constexpr int kChunk = 32;
+
+B2G_DEV int Uniform( int x )
+{
+	return __builtin_amdgcn_readfirstlane( x );
+}
+
+// What a workgroup keeps of its world's arguments in registers, and where each lane stands.
+struct FusedLane
+{
+	ConstraintSoA c;
+	const int* bodies; // the lane's side's slots
+	int wave;  // this lane's wavefront
+	int waves; // a power of two
+	int pair;  // constraint within a chunk
+	int side;  // 0: body A, 1: body B
+	int colors;
+	int contactStarts; // lane k: first contact of color k (lane `colors`: the end)
+	int jointStarts;   // the same for joints
+	bool anyJoints;
+	float inv_h;
+	float contactSpeed;
+};
+
+// The wavefront's place in a stage's sequence of contact chunks; color == colors after the last one.
+struct ChunkCursor
+{
+	int color;
+	int start; // first constraint
+	int count; // constraints
+	int chunk; // number within its color
+	int base;  // chunks of the colors before
+};
+
+// Move to the first chunk of this wavefront at or after q.chunk of q.color.
+B2G_DEV void SeekChunk( const FusedLane& L, ChunkCursor& q )
+{
+	q.count = 0;
+	while ( q.color < L.colors )
+	{
+		int begin = __builtin_amdgcn_readlane( L.contactStarts, q.color );
+		int lanes = __builtin_amdgcn_readlane( L.contactStarts, q.color + 1 ) - begin;
+		if ( kChunk * q.chunk < lanes )
+		{
+			q.start = begin + kChunk * q.chunk;
+			q.count = Uniform( b2MinInt( kChunk, lanes - kChunk * q.chunk ) );
+			return;
+		}
+		q.base += ( lanes + kChunk - 1 ) / kChunk;
+		q.color = Uniform( q.color + 1 );
+		q.chunk = Uniform( ( L.wave - q.base ) & ( L.waves - 1 ) );
+	}
+}
+
+B2G_DEV void FirstChunk( const FusedLane& L, ChunkCursor& q )
+{
+	q.color = 0;
+	q.start = 0;
+	q.base = 0;
+	q.chunk = L.wave;
+	SeekChunk( L, q );
+}
+
+// A chunk in hand: its rows (loaded or on their way) and the lane's own body.
+struct ChunkRow
+{
+	PairRow row;
+	int slot;
+};
+
+// Lanes without a constraint load the chunk's last one (an empty chunk the row at q.start, which
+// every allocation holds), so that the loads go straight into the loop's registers.
+template <int Stage>
+B2G_DEV void LoadChunk( const FusedLane& L, const ChunkCursor& q, ChunkRow& r )
+{
+	int i = q.start + b2MinInt( L.pair, b2MaxInt( q.count - 1, 0 ) );
+	r.slot = L.bodies[i];
+	LoadPairRow<Stage>( L.c, i, L.side, r.row );
+}
+
+// Waits for a loaded row where its turn begins: what is computed from it cannot be moved up to its
+// loads, where it would make the wavefront wait for them before the barriers in between.
+template <int Stage>
+B2G_DEV void AwaitChunk( ChunkRow& r )
+{
+	PairRow& x = r.row;
+	asm volatile( "" : "+v"( r.slot ), "+v"( x.mass ), "+v"( x.normal ), "+v"( x.a1 ), "+v"( x.a2 ),
+				  "+v"( x.i1 ), "+v"( x.i2 ) );
+	if ( Stage == kStageSolve )
+	{
+		asm volatile( "" : "+v"( x.soft ), "+v"( x.m1 ), "+v"( x.m2 ) );
+	}
+	else if ( Stage == kStageRelax )
+	{
+		asm volatile( "" : "+v"( x.rolling ), "+v"( x.m1 ), "+v"( x.m2 ) );
+	}
+	else
+	{
+		asm volatile( "" : "+v"( x.rolling ) );
+	}
+}
+
+template <int Stage>
+B2G_DEV RowBias ChunkBias( const FusedLane& L, const PackedBodies& B, const ChunkRow& r )
+{
+	const float4 d = B.d[r.slot];
+	return ComputePairBias<Stage == kStageSolve>( r.row, F4{ d.x, d.y, d.z, d.w }, L.inv_h, L.contactSpeed );
+}
+
+// One stage's work on the constraint of a lane pair.
+template <int Stage>
+B2G_DEV void SolveChunk( const PackedBodies& B, ChunkRow& r, F2 mass, bool dynamic, const RowBias& bias, bool* rolling )
+{
+	float* own = B.v + 3 * r.slot;
+	OwnVel v = { own[0], own[1], own[2] };
+	if ( Stage == kStageWarmStart )
+	{
+		WarmStartPair( r.row, mass, v );
+	}
+	else if ( Stage == kStageSolve )
+	{
+		SolvePair<true>( r.row, mass, v, bias, false );
+	}
+	else
+	{
+		// a group of four constraints is eight neighbouring lanes
+		unsigned long long any = __ballot( r.row.rolling.x != 0.0f );
+		*rolling = ( ( any >> ( threadIdx.x & 56 ) ) & 0xFF ) != 0;
+		SolvePair<false>( r.row, mass, v, bias, *rolling );
+	}
+	if ( dynamic )
+	{
+		own[0] = v.x;
+		own[1] = v.y;
+		own[2] = v.w;
+	}
+}
+
+B2G_DEV void StoreChunk( const FusedLane& L, const ChunkCursor& q, const ChunkRow& r, bool rolling )
+{
+	int i = q.start + L.pair;
+	StorePairImpulses( L.c, i, L.side, r.row );
+	if ( rolling && L.side == 0 )
+	{
+		L.c.f[kcRollingImpulse][i] = r.row.rolling.z;
+	}
+}
+
+B2G_DEV F2 SignedMass( const FusedLane& L, F2 mass )
+{
+	return L.side == 0 ? -mass : mass;
+}
+
+B2G_DEV int ColorContacts( const FusedLane& L, int color )
+{
+	return __builtin_amdgcn_readlane( L.contactStarts, color + 1 ) - __builtin_amdgcn_readlane( L.contactStarts, color );
+}
+
+// One stage over the colors, with the rows of the wavefront's first chunk on their way. At the end
+// those of its first chunk of NextStage are (unless `prefetchNext` is false).
+template <bool kGeneral, int Stage, int NextStage>
+B2G_DEV void FusedContactStage( const FusedArgs& a, const FusedLane& L, const PackedBodies& B, ChunkCursor& q, ChunkRow& r,
+								bool prefetchNext )
+{
+	if ( kGeneral && ( a.overflowContactCount > 0 || a.overflowJointCount > 0 ) )
+	{
+		if ( threadIdx.x == 0 )
+		{
+			ColorRange range = { a.overflowJointStart, a.overflowJointCount, a.overflowContactStart, a.overflowContactCount };
+			OverflowSerial<Stage>( a.color, range, B );
+		}
+		LdsBarrier();
+	}
+
+	// The loop runs over the wavefront's chunks and passes the colors in between, so that a chunk's
+	// rows are loaded in one place, straight into the registers the next turn reads.
+	int color = 0;
+	int jointBase = L.waves >> 1;
+	auto passColor = [&]() {
+		int lanes = ColorContacts( L, color );
+		if ( kGeneral && L.anyJoints )
+		{
+			int jointStart = __builtin_amdgcn_readlane( L.jointStarts, color );
+			int joints = __builtin_amdgcn_readlane( L.jointStarts, color + 1 ) - jointStart;
+			for ( int k = ( L.wave - jointBase ) & ( L.waves - 1 ); 64 * k < joints; k += L.waves )
+			{
+				ColorRange range = { jointStart, joints, 0, 0 };
+				ColorLane<Stage>( a.color, range, 64 * k + ( threadIdx.x & 63 ), B );
+			}
+			jointBase += ( joints + 63 ) >> 6;
+			lanes += joints;
+		}
+		if ( lanes > 0 )
+		{
+			LdsBarrier();
+		}
+		color = Uniform( color + 1 );
+	};
+	bool more = Uniform( q.color ) < L.colors;
+	while ( more )
+	{
+		while ( color < Uniform( q.color ) )
+		{
+			passColor();
+		}
+		AwaitChunk<Stage>( r );
+		if ( L.pair < q.count )
+		{
+			RowBias bias;
+			if ( Stage != kStageWarmStart )
+			{
+				bias = ChunkBias<Stage>( L, B, r );
+			}
+			bool rolling = false;
+			bool dynamic = ( B.flags[r.slot] & kDynamicFlag ) != 0;
+			SolveChunk<Stage>( B, r, SignedMass( L, r.row.mass ), dynamic, bias, &rolling );
+			StoreChunk( L, q, r, rolling );
+		}
+		q.chunk += L.waves;
+		SeekChunk( L, q );
+		more = Uniform( q.color ) < L.colors;
+		if ( Uniform( q.color ) != color )
+		{
+			passColor();
+		}
+		if ( more == false )
+		{
+			break;
+		}
+		LoadChunk<Stage>( L, q, r );
+	}
+	while ( color < L.colors )
+	{
+		passColor();
+	}
+	FirstChunk( L, q );
+	if ( prefetchNext )
+	{
+		LoadChunk<NextStage>( L, q, r );
+	}
+}
+
+// Worlds whose contact chunks number at most kResidentRows per wavefront keep every row in registers.
+constexpr int kResidentRows = 2;
+
+struct ResidentChunks
+{
+	ChunkCursor q[kResidentRows];
+	ChunkRow r[kResidentRows];
+	F2 mass[kResidentRows];
+	bool active[kResidentRows];	 // this lane pair has a constraint
+	bool dynamic[kResidentRows]; // its own body moves
+};
+
+B2G_DEV void LoadResident( const FusedLane& L, ResidentChunks& R )
+{
+	ChunkCursor q;
+	FirstChunk( L, q );
+#pragma unroll
+	for ( int k = 0; k < kResidentRows; ++k )
+	{
+		R.q[k] = q;
+		R.active[k] = L.pair < q.count;
+		R.r[k].slot = kStaticSlot;
+		if ( Uniform( q.count ) > 0 )
+		{
+			LoadChunk<kStageRelax>( L, q, R.r[k] );
+			R.r[k].row.soft = PairGroup( L.c, kgSoft, q.start + b2MinInt( L.pair, q.count - 1 ) );
+			R.mass[k] = SignedMass( L, R.r[k].row.mass );
+		}
+		q.chunk += L.waves;
+		SeekChunk( L, q );
+	}
+}
+
+template <int Stage>
+B2G_DEV void ResidentStage( const FusedLane& L, const PackedBodies& B, ResidentChunks& R, bool store )
+{
+	RowBias bias[kResidentRows];
+	if ( Stage != kStageWarmStart )
+	{
+#pragma unroll
+		for ( int k = 0; k < kResidentRows; ++k )
+		{
+			if ( R.active[k] )
+			{
+				bias[k] = ChunkBias<Stage>( L, B, R.r[k] );
+			}
+		}
+	}
+	for ( int color = 0; color < L.colors; ++color )
+	{
+		if ( ColorContacts( L, color ) == 0 )
+		{
+			continue;
+		}
+#pragma unroll
+		for ( int k = 0; k < kResidentRows; ++k )
+		{
+			if ( Uniform( R.q[k].color ) == color && R.active[k] )
+			{
+				bool rolling = false;
+				SolveChunk<Stage>( B, R.r[k], R.mass[k], R.dynamic[k], bias[k], &rolling );
+				if ( store )
+				{
+					StoreChunk( L, R.q[k], R.r[k], rolling );
+				}
+			}
+		}
+		LdsBarrier();
+	}
+}
+
+// The restitution stage, once per step and only for worlds with restitution.
+B2G_DEV void FusedRestitution( const FusedArgs& a, const PackedBodies& B )
+{
+	if ( ( a.overflowContactCount > 0 || a.overflowJointCount > 0 ) && threadIdx.x == 0 )
+	{
+		ColorRange r = { a.overflowJointStart, a.overflowJointCount, a.overflowContactStart, a.overflowContactCount };
+		OverflowSerial<kStageRestitution>( a.color, r, B );
+	}
+	__syncthreads();
+	for ( int color = 0; color < a.activeColorCount; ++color )
+	{
+		ColorRange r = { 0, 0, a.colorContactStart[color], a.colorContactStart[color + 1] - a.colorContactStart[color] };
+		for ( int t = threadIdx.x; t < r.contactCount; t += blockDim.x )
+		{
+			ColorLane<kStageRestitution>( a.color, r, t, B );
+		}
+		__syncthreads();
+	}
+}
+
+// Bodies per lane whose velocity-integration terms stay in registers over the substeps.
+constexpr int kFusedBodyRegs = 2;
+
+// Forms of the fused solver. General: joints, overflow constraints, restitution, the body-by-body
+// warm start. Streamed and resident leave that code out, and with it the registers it takes from the
+// contact rows.
+enum FusedForm
+{
+	kFusedGeneral,
+	kFusedStreamed,
+	kFusedResident,
+};
+
+__host__ __device__ inline bool FusedIsGeneral( const FusedArgs& a )
+{
+	return a.colorJointStart[a.activeColorCount] > a.colorJointStart[0] || a.overflowContactCount > 0 || a.overflowJointCount > 0 ||
+		   a.anyRestitution != 0 || a.warmByBody != 0;
+}
+
+// The whole substep loop of one world by the calling workgroup (a power of two of wavefronts), body
+// states in the dynamic LDS at lds.
+template <int kForm>
 B2G_DEV void FusedBody( const FusedArgs& a, char* lds )
 {
+	constexpr bool kGeneral = kForm == kFusedGeneral;
+	constexpr bool kResident = kForm == kFusedResident;
+	const bool warmByBody = kGeneral && a.warmByBody != 0;
 	const int n = a.bodyCount;
 	const int cap = n + 1;
-	float* s_vx = reinterpret_cast<float*>( lds );
-	float* s_vy = s_vx + cap;
-	float* s_w = s_vy + cap;
-	float* s_dpx = s_w + cap;
-	float* s_dpy = s_dpx + cap;
-	float* s_dqc = s_dpy + cap;
-	float* s_dqs = s_dqc + cap;
-	uint16_t* s_flags = reinterpret_cast<uint16_t*>( s_dqs + cap );
-
-	LdsBodies B{ s_vx, s_vy, s_w, s_dpx, s_dpy, s_dqc, s_dqs, s_flags };
+	PackedBodies B;
+	B.d = reinterpret_cast<float4*>( lds );
+	B.v = reinterpret_cast<float*>( B.d + cap );
+	B.flags = reinterpret_cast<uint16_t*>( B.v + 3 * cap );
 	const GlobalBodies G{ a.states };
+	const StepParams& p = a.color.p;
 
-	auto put = [&]( int slot, const BodyState& st ) {
-		s_vx[slot] = st.linearVelocity.x;
-		s_vy[slot] = st.linearVelocity.y;
-		s_w[slot] = st.angularVelocity;
-		s_flags[slot] = (uint16_t)st.flags;
-		s_dpx[slot] = st.deltaPosition.x;
-		s_dpy[slot] = st.deltaPosition.y;
-		s_dqc[slot] = st.deltaRotation.c;
-		s_dqs[slot] = st.deltaRotation.s;
+	FusedLane L;
+	L.c = a.color.c;
+	L.wave = Uniform( threadIdx.x >> 6 );
+	L.waves = Uniform( blockDim.x >> 6 );
+	L.pair = ( threadIdx.x & 63 ) >> 1;
+	L.side = threadIdx.x & 1;
+	L.bodies = L.side == 0 ? L.c.bodyA : L.c.bodyB;
+	L.colors = Uniform( a.activeColorCount );
+	{
+		const int k = b2MinInt( threadIdx.x & 63, L.colors );
+		L.contactStarts = a.colorContactStart[k];
+		L.jointStarts = a.colorJointStart[k];
+		// these loads are waited for here, not at each use among the rows' loads in flight
+		asm volatile( "" : "+v"( L.contactStarts ), "+v"( L.jointStarts ) );
+	}
+	L.anyJoints = a.colorJointStart[L.colors] > a.colorJointStart[0];
+	L.inv_h = p.inv_h;
+	L.contactSpeed = -p.contactSpeed;
+
+	// the first rows on their way
+	ChunkCursor q;
+	ChunkRow r;
+	ResidentChunks R;
+	if ( kResident )
+	{
+		LoadResident( L, R );
+	}
+	else
+	{
+		FirstChunk( L, q );
+		if ( warmByBody == false )
+		{
+			LoadChunk<kStageWarmStart>( L, q, r );
+		}
+	}
+
+	VelocityStep vs[kFusedBodyRegs];
+#pragma unroll
+	for ( int k = 0; k < kFusedBodyRegs; ++k )
+	{
+		int i = threadIdx.x + k * blockDim.x;
+		if ( i < n )
+		{
+			vs[k] = MakeVelocityStep( a.sims[a.awake[i]], p );
+		}
+	}
+	auto put = [&]( int slot, const LaneBody& st ) {
+		B.d[slot] = make_float4( st.dpx, st.dpy, st.dqc, st.dqs );
+		B.StoreVelocity( slot, st.vx, st.vy, st.w );
+		B.flags[slot] = (uint16_t)st.flags;
 	};
-
 	for ( int i = threadIdx.x; i < n; i += blockDim.x )
 	{
-		put( i + 1, ToState( G.Load( a.awake[i] ) ) );
+		put( i + 1, G.Load( a.awake[i] ) );
 	}
 	if ( threadIdx.x == 0 )
 	{
 		// identity state of static bodies (reference b2_identityBodyState)
-		BodyState id;
-		id.linearVelocity = { 0.0f, 0.0f };
-		id.angularVelocity = 0.0f;
-		id.flags = 0;
-		id.deltaPosition = { 0.0f, 0.0f };
-		id.deltaRotation = { 1.0f, 0.0f };
-		put( kStaticSlot, id );
+		put( kStaticSlot, LaneBody{ 0.0f, 0.0f, 0.0f, 0, 0.0f, 0.0f, 1.0f, 0.0f } );
 	}
-	__syncthreads();
+	LdsBarrier();
+	if ( kResident )
+	{
+#pragma unroll
+		for ( int k = 0; k < kResidentRows; ++k )
+		{
+			R.dynamic[k] = ( B.flags[R.r[k].slot] & kDynamicFlag ) != 0;
+		}
+	}
+
+	auto integrateVelocity = [&]( int i, const VelocityStep& step ) {
+		float* bv = B.v + 3 * ( i + 1 );
+		b2Vec2 v = { bv[0], bv[1] };
+		float w = bv[2];
+		ApplyVelocityStep( step, v, w );
+		B.StoreVelocity( i + 1, v.x, v.y, w );
+	};
 
 	for ( int sub = 0; sub < a.subStepCount; ++sub )
 	{
-		// velocity integration, then the warm-start stage color by color or body by body (one
-		// barrier instead of one per color; the floats are the same either way)
-		for ( int i = threadIdx.x; i < n; i += blockDim.x )
+		const bool last = sub + 1 == a.subStepCount;
+		// velocity integration, then the warm-start stage color by color or body by body (the floats
+		// are the same either way)
+#pragma unroll
+		for ( int k = 0; k < kFusedBodyRegs; ++k )
 		{
-			BodyState st = ToState( B.Load( i + 1 ) );
-			IntegrateVelocity( a.sims[a.awake[i]], &st, a.color.p );
-			float vx = st.linearVelocity.x, vy = st.linearVelocity.y, w = st.angularVelocity;
-			if ( a.warmByBody )
+			int i = threadIdx.x + k * blockDim.x;
+			if ( i < n )
 			{
-				WarmStartBody( a.color.c, a.color.joints, a.color.jointList, a.overflowContactStart, a.warmList, a.warmStart[i],
-							   a.warmStart[i + 1], B, st.deltaRotation, st.deltaPosition, vx, vy, w );
+				integrateVelocity( i, vs[k] );
 			}
-			s_vx[i + 1] = vx;
-			s_vy[i + 1] = vy;
-			s_w[i + 1] = w;
 		}
-		__syncthreads();
-
-		if ( a.warmByBody == 0 )
+		for ( int i = threadIdx.x + kFusedBodyRegs * blockDim.x; i < n; i += blockDim.x )
 		{
-			FusedStage<kStageWarmStart>( a, B );
+			integrateVelocity( i, MakeVelocityStep( a.sims[a.awake[i]], p ) );
 		}
-		FusedStage<kStageSolve>( a, B );
+		if ( warmByBody )
+		{
+			__syncthreads(); // other lanes' impulses and joint rows are read below
+			for ( int i = threadIdx.x; i < n; i += blockDim.x )
+			{
+				LaneBody st = B.Load( i + 1 );
+				WarmStartBody( L.c, a.color.joints, a.color.jointList, a.overflowContactStart, a.warmList, a.warmStart[i],
+							   a.warmStart[i + 1], B, b2Rot{ st.dqc, st.dqs }, b2Vec2{ st.dpx, st.dpy }, st.vx, st.vy, st.w );
+				B.StoreVelocity( i + 1, st.vx, st.vy, st.w );
+			}
+			__syncthreads();
+			LoadChunk<kStageSolve>( L, q, r );
+		}
+		else
+		{
+			LdsBarrier();
+			if ( kResident )
+			{
+				ResidentStage<kStageWarmStart>( L, B, R, false );
+			}
+			else
+			{
+				FusedContactStage<kGeneral, kStageWarmStart, kStageSolve>( a, L, B, q, r, true );
+			}
+		}
+		if ( kResident )
+		{
+			ResidentStage<kStageSolve>( L, B, R, false );
+		}
+		else
+		{
+			FusedContactStage<kGeneral, kStageSolve, kStageRelax>( a, L, B, q, r, true );
+		}
 
 		for ( int i = threadIdx.x; i < n; i += blockDim.x )
 		{
 			BodyState st = ToState( B.Load( i + 1 ) );
-			IntegratePosition( &st, a.color.p );
-			put( i + 1, st );
+			IntegratePosition( &st, p );
+			put( i + 1, ToLane( st ) );
 		}
-		__syncthreads();
+		LdsBarrier();
 
-		FusedStage<kStageRelax>( a, B );
+		if ( kResident )
+		{
+			ResidentStage<kStageRelax>( L, B, R, last );
+		}
+		else
+		{
+			FusedContactStage<kGeneral, kStageRelax, kStageWarmStart>( a, L, B, q, r, warmByBody == false && last == false );
+		}
 	}
 
-	if ( a.anyRestitution )
+	if ( kGeneral && a.anyRestitution )
 	{
-		FusedStage<kStageRestitution>( a, B );
+		__syncthreads();
+		FusedRestitution( a, B );
 	}
 
 	// write the whole state back (flags carry the speed-cap bit to finalize)
 	for ( int i = threadIdx.x; i < n; i += blockDim.x )
 	{
+		LaneBody st = B.Load( i + 1 );
 		BodyState* dst = a.states + a.awake[i];
-		dst->linearVelocity = { s_vx[i + 1], s_vy[i + 1] };
-		dst->angularVelocity = s_w[i + 1];
-		dst->flags = ( dst->flags & 0xFFFF0000u ) | s_flags[i + 1];
-		dst->deltaPosition = { s_dpx[i + 1], s_dpy[i + 1] };
-		dst->deltaRotation = { s_dqc[i + 1], s_dqs[i + 1] };
+		dst->linearVelocity = { st.vx, st.vy };
+		dst->angularVelocity = st.w;
+		dst->flags = ( dst->flags & 0xFFFF0000u ) | st.flags;
+		dst->deltaPosition = { st.dpx, st.dpy };
+		dst->deltaRotation = { st.dqc, st.dqs };
 	}
 }
 
-__global__ __launch_bounds__( kFusedThreads ) void SolveFusedKernel( FusedArgs a )
+// The general form gets twice the registers and half the threads.
+constexpr int kFusedGeneralThreads = 512;
+
+template <int kForm>
+__global__ __launch_bounds__( kForm == kFusedGeneral ? kFusedGeneralThreads : kFusedThreads ) void SolveFusedKernel( FusedArgs a )
 {
-	extern __shared__ char s_lds[];
-	FusedBody( a, s_lds );
+	extern __shared__ __align__( 16 ) char s_lds[];
+	FusedBody<kForm>( a, s_lds );
+}
+
+// Form and threads of a single world's fused solve: a wavefront per chunk of a stage's constraints, up
+// to the form's limit; resident when all chunks fit.
+static FusedForm FusedPlan( const FusedArgs& a, int* threads )
+{
+	int chunks = 0;
+	for ( int c = 0; c < a.activeColorCount; ++c )
+	{
+		chunks += ( a.colorContactStart[c + 1] - a.colorContactStart[c] + kChunk - 1 ) / kChunk +
+				  ( a.colorJointStart[c + 1] - a.colorJointStart[c] + 63 ) / 64;
+	}
+	const FusedForm form = FusedIsGeneral( a ) ? kFusedGeneral
+						   : chunks <= kResidentRows * kFusedThreads / 64 ? kFusedResident
+																		  : kFusedStreamed;
+	const int most = form == kFusedGeneral ? kFusedGeneralThreads : kFusedThreads;
+	*threads = 64;
+	while ( *threads < most && *threads < 64 * chunks )
+	{
+		*threads *= 2;
+	}
+	return form;
 }
 
 // Persistent form over many worlds: each workgroup takes the next world from a queue (worlds
 // ordered largest first) until the queue is empty. Every workgroup reaches the queue's end, so
 // the launch drains without any inter-group wait.
-__global__ __launch_bounds__( kFusedThreads ) void SolveFusedBatchKernel( const FusedArgs* args, const int* order, int count,
-																		  int* queue )
+template <int kThreads>
+__global__ __launch_bounds__( kThreads ) void SolveFusedBatchKernel( const FusedArgs* args, const int* order, int count, int* queue )
 {
-	extern __shared__ char s_lds[];
+	extern __shared__ __align__( 16 ) char s_lds[];
 	__shared__ int s_world;
 	for ( ;; )
 	{
@@ -1422,7 +1850,15 @@ __global__ __launch_bounds__( kFusedThreads ) void SolveFusedBatchKernel( const 
 			break;
 		}
 		int world = __builtin_amdgcn_readfirstlane( order[w] );
-		FusedBody( args[world], s_lds );
+		const FusedArgs& a = args[world];
+		if ( FusedIsGeneral( a ) )
+		{
+			FusedBody<kFusedGeneral>( a, s_lds );
+		}
+		else
+		{
+			FusedBody<kFusedStreamed>( a, s_lds );
+		}
 		__syncthreads();
 	}
 }
@@ -1672,11 +2108,11 @@ B2G_DEV void StoreImpulsesBody( const StoreArgs& a, int i )
 
 	for ( int j = 0; j < writeCount; ++j )
 	{
-		int o = j == 0 ? 0 : ( kcAnchorA2X - kcAnchorA1X );
-		m->points[j].normalImpulse = c.f[kcNormalImpulse1 + o][i];
-		m->points[j].tangentImpulse = c.f[kcTangentImpulse1 + o][i];
-		m->points[j].totalNormalImpulse = c.f[kcTotalNormalImpulse1 + o][i];
-		m->points[j].normalVelocity = c.f[kcRelativeVelocity1 + o][i];
+		const float4 impulse = c.f.Group( j == 0 ? kgImpulse1 : kgImpulse2 )[i];
+		m->points[j].normalImpulse = impulse.x;
+		m->points[j].tangentImpulse = impulse.y;
+		m->points[j].totalNormalImpulse = impulse.z;
+		m->points[j].normalVelocity = c.f[j == 0 ? kcRelativeVelocity1 : kcRelativeVelocity2][i];
 	}
 	m->rollingImpulse = c.f[kcRollingImpulse][i];
 
@@ -3267,10 +3703,15 @@ static void EnableLargeLds()
 				(void)hipGetLastError();
 			}
 		}
-		HIP_CHECK( hipFuncSetAttribute( reinterpret_cast<const void*>( SolveFusedKernel ),
-										hipFuncAttributeMaxDynamicSharedMemorySize, FusedLdsBytes( kFusedBodyCapacity ) ) );
-		HIP_CHECK( hipFuncSetAttribute( reinterpret_cast<const void*>( SolveFusedBatchKernel ),
-										hipFuncAttributeMaxDynamicSharedMemorySize, FusedLdsBytes( kFusedBodyCapacity ) ) );
+		const void* fusedKernels[5] = { reinterpret_cast<const void*>( SolveFusedKernel<kFusedGeneral> ),
+										reinterpret_cast<const void*>( SolveFusedKernel<kFusedStreamed> ),
+										reinterpret_cast<const void*>( SolveFusedKernel<kFusedResident> ),
+										reinterpret_cast<const void*>( SolveFusedBatchKernel<512> ),
+										reinterpret_cast<const void*>( SolveFusedBatchKernel<1024> ) };
+		for ( const void* k : fusedKernels )
+		{
+			HIP_CHECK( hipFuncSetAttribute( k, hipFuncAttributeMaxDynamicSharedMemorySize, FusedLdsBytes( kFusedBodyCapacity ) ) );
+		}
 		const void* overflowKernels[4] = { reinterpret_cast<const void*>( OverflowLevelKernel<kStageWarmStart> ),
 										   reinterpret_cast<const void*>( OverflowLevelKernel<kStageSolve> ),
 										   reinterpret_cast<const void*>( OverflowLevelKernel<kStageRelax> ),
@@ -4800,7 +5241,14 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 		}
 		else
 		{
-			impl->Launch( kkSolveFused, bytes, [&]( hipEvent_t e0, hipEvent_t e1 ) { hipExtLaunchKernelGGL( SolveFusedKernel, dim3( 1 ), dim3( kFusedThreads ), FusedLdsBytes( nb ), s, e0, e1, 0, fa ); } );
+			int threads = 0;
+			const FusedForm form = FusedPlan( fa, &threads );
+			const auto kernel = form == kFusedGeneral ? SolveFusedKernel<kFusedGeneral>
+								: form == kFusedStreamed ? SolveFusedKernel<kFusedStreamed>
+														 : SolveFusedKernel<kFusedResident>;
+			impl->Launch( kkSolveFused, bytes, [&]( hipEvent_t e0, hipEvent_t e1 ) {
+				hipExtLaunchKernelGGL( kernel, dim3( 1 ), dim3( threads ), FusedLdsBytes( nb ), s, e0, e1, 0, fa );
+			} );
 		}
 	}
 	else
@@ -6069,11 +6517,12 @@ void Batch::Solve( DeviceWorld** worlds, int count )
 		const int threads = BatchTuningFor( most ).threads;
 		int lds = FusedLdsBytes( fusedBodies[order[0]] );
 		int perCu = 0;
-		HIP_CHECK( hipOccupancyMaxActiveBlocksPerMultiprocessor( &perCu, SolveFusedBatchKernel, threads, lds ) );
+		const auto kernel = threads > 512 ? SolveFusedBatchKernel<1024> : SolveFusedBatchKernel<512>;
+		HIP_CHECK( hipOccupancyMaxActiveBlocksPerMultiprocessor( &perCu, kernel, threads, lds ) );
 		int grid = std::max( 1, std::min( total, perCu * b->cuCount ) );
 		HIP_CHECK( hipMemsetAsync( b->queue, 0, sizeof( int ), s ) );
 		// the events bracket the kernel's execution (recorded by the dispatch itself)
-		hipExtLaunchKernelGGL( SolveFusedBatchKernel, dim3( grid ), dim3( threads ), (uint32_t)lds, s, b->ev0, b->ev1, 0,
+		hipExtLaunchKernelGGL( kernel, dim3( grid ), dim3( threads ), (uint32_t)lds, s, b->ev0, b->ev1, 0,
 							   reinterpret_cast<const FusedArgs*>( base + fusedOff ), reinterpret_cast<const int*>( base + orderOff ),
 							   total, b->queue );
 		HIP_CHECK( hipGetLastError() );

@@ -7,8 +7,8 @@
 // "dummy state" the reference substitutes for a null solver index (src/body.h:165), so solver
 // lanes never branch on null bodies.
 //
-// Contact constraints are stored structure-of-arrays (one float array per field) so a wavefront
-// reads each field with one coalesced load; the fields are those of b2ContactConstraintWide
+// Contact constraints are stored as one array per group of four fields, so a wavefront reads a
+// constraint's rows with coalesced 16-byte loads; the fields are those of b2ContactConstraintWide
 // (reference src/contact_solver.c:1070-1100).
 #pragma once
 
@@ -284,46 +284,56 @@ struct JointSim
 	int pad;
 };
 
-// Contact constraint fields, one device array per field (structure of arrays).
+// Contact constraint fields, in groups of four that a lane loads as one float4 (see RowTable). The
+// fields of point 2 follow those of point 1 at one distance, kcAnchorA2X - kcAnchorA1X.
 enum ConstraintField
 {
+	// group 0: masses, a pair per body
 	kcInvMassA,
-	kcInvMassB,
 	kcInvIA,
+	kcInvMassB,
 	kcInvIB,
+	// group 1: normal and friction
 	kcNormalX,
 	kcNormalY,
 	kcFriction,
 	kcTangentSpeed,
-	kcRollingResistance,
-	kcRollingMass,
-	kcRollingImpulse,
+	// group 2: softness
 	kcBiasRate,
 	kcMassScale,
 	kcImpulseScale,
 	kcRestitution,
+	// group 3: rolling
+	kcRollingResistance,
+	kcRollingMass,
+	kcRollingImpulse,
+	kcPadRolling,
+	// groups 4-6: point 1 (anchors; separation and masses; what the solver writes)
 	kcAnchorA1X,
 	kcAnchorA1Y,
 	kcAnchorB1X,
 	kcAnchorB1Y,
 	kcBaseSeparation1,
-	kcNormalImpulse1,
-	kcTangentImpulse1,
-	kcTotalNormalImpulse1,
 	kcNormalMass1,
 	kcTangentMass1,
 	kcRelativeVelocity1,
+	kcNormalImpulse1,
+	kcTangentImpulse1,
+	kcTotalNormalImpulse1,
+	kcPadImpulse1,
+	// groups 7-9: point 2
 	kcAnchorA2X,
 	kcAnchorA2Y,
 	kcAnchorB2X,
 	kcAnchorB2Y,
 	kcBaseSeparation2,
-	kcNormalImpulse2,
-	kcTangentImpulse2,
-	kcTotalNormalImpulse2,
 	kcNormalMass2,
 	kcTangentMass2,
 	kcRelativeVelocity2,
+	kcNormalImpulse2,
+	kcTangentImpulse2,
+	kcTotalNormalImpulse2,
+	kcPadImpulse2,
 	kcFieldCount
 };
 

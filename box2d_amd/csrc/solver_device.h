@@ -18,8 +18,7 @@ namespace b2g
 
 #define B2G_DEVI __device__ __forceinline__
 
-// The constraint fields live in one allocation, field-major: field k of constraint i is at
-// base[k * stride + i]. f[k] yields the field's array, so lanes read c.f[k][i].
+// Float arrays of one allocation, field-major: field k of element i is at base[k * stride + i].
 struct FieldTable
 {
 	float* base;
@@ -31,14 +30,47 @@ struct FieldTable
 	}
 };
 
+// One field of a RowTable.
+struct RowField
+{
+	float* p;
+
+	__host__ __device__ float& operator[]( int i ) const
+	{
+		return p[4 * (size_t)i];
+	}
+	__host__ __device__ float* operator+( int i ) const
+	{
+		return p + 4 * (size_t)i;
+	}
+};
+
+// The constraint fields (ConstraintField): one allocation, one float4 array of `stride` constraints
+// per group of four fields. A lane loads the groups a stage needs with 7 to 9 16-byte loads instead
+// of about 30 4-byte ones. table[k][i] is field k of constraint i; Group( g )[i] is group g's four.
+struct RowTable
+{
+	float* base;
+	int stride;
+
+	__host__ __device__ RowField operator[]( int field ) const
+	{
+		return RowField{ base + 4 * (size_t)( field >> 2 ) * stride + ( field & 3 ) };
+	}
+	__host__ __device__ float4* Group( int group ) const
+	{
+		return reinterpret_cast<float4*>( base ) + (size_t)group * stride;
+	}
+};
+
 struct ConstraintSoA
 {
-	FieldTable f;
+	RowTable f;
 	int* bodyA; // body ids (GlobalBodies view)
 	int* bodyB;
 	int* contactId;
 	int* pointCount;
-	int* slotA; // LDS slots of the fused solver (LdsBodies view)
+	int* slotA; // LDS slots of the fused solver (LdsBodies, PackedBodies views)
 	int* slotB;
 };
 
@@ -298,28 +330,96 @@ struct LdsBodies
 	}
 };
 
+// A world's awake bodies in LDS as the fused solver keeps them: the delta pose as one 16-byte word,
+// the velocity as three floats (12 bytes, so that neighbouring slots fall into different banks) and
+// the flags, 30 bytes per slot.
+struct PackedBodies
+{
+	float4* d;
+	float* v;
+	uint16_t* flags;
+
+	B2G_DEVI LaneBody Load( int index ) const
+	{
+		float4 p = d[index];
+		LaneBody r;
+		r.vx = v[3 * index];
+		r.vy = v[3 * index + 1];
+		r.w = v[3 * index + 2];
+		r.flags = flags[index];
+		r.dpx = p.x;
+		r.dpy = p.y;
+		r.dqc = p.z;
+		r.dqs = p.w;
+		return r;
+	}
+
+	B2G_DEVI void LoadDelta( int index, b2Vec2& dp, b2Rot& dq ) const
+	{
+		float4 p = d[index];
+		dp = { p.x, p.y };
+		dq = { p.z, p.w };
+	}
+
+	B2G_DEVI void StoreVelocity( int index, float vx, float vy, float w ) const
+	{
+		v[3 * index] = vx;
+		v[3 * index + 1] = vy;
+		v[3 * index + 2] = w;
+	}
+
+	B2G_DEVI void Store( int index, const LaneBody& b ) const
+	{
+		if ( b.flags & kDynamicFlag )
+		{
+			StoreVelocity( index, b.vx, b.vy, b.w );
+		}
+	}
+
+	B2G_DEVI static int JointA( const JointSim* j )
+	{
+		return j->slotA;
+	}
+	B2G_DEVI static int JointB( const JointSim* j )
+	{
+		return j->slotB;
+	}
+};
+
 // ---------------------------------------------------------------------------------------------
 // Body integration
 
+// What velocity integration adds and multiplies, the same in every substep of a step.
+struct VelocityStep
+{
+	b2Vec2 linearVelocityDelta;
+	float linearDamping;
+	float angularVelocityDelta;
+	float angularDamping;
+};
+
+B2G_DEVI VelocityStep MakeVelocityStep( const BodySim& sim, const StepParams& p )
+{
+	float h = p.h;
+	VelocityStep s;
+	s.linearDamping = 1.0f / ( 1.0f + h * sim.linearDamping );
+	s.angularDamping = 1.0f / ( 1.0f + h * sim.angularDamping );
+	float gravityScale = sim.invMass > 0.0f ? sim.gravityScale : 0.0f;
+	s.linearVelocityDelta = b2Add( b2MulSV( h * sim.invMass, sim.force ), b2MulSV( h * gravityScale, p.gravity ) );
+	s.angularVelocityDelta = h * sim.invInertia * sim.torque;
+	return s;
+}
+
 // Velocity integration of one body (reference src/solver.c:66-112).
+B2G_DEVI void ApplyVelocityStep( const VelocityStep& s, b2Vec2& v, float& w )
+{
+	v = b2MulAdd( s.linearVelocityDelta, s.linearDamping, v );
+	w = s.angularVelocityDelta + s.angularDamping * w;
+}
+
 B2G_DEVI void IntegrateVelocity( const BodySim& sim, BodyState* state, const StepParams& p )
 {
-	b2Vec2 v = state->linearVelocity;
-	float w = state->angularVelocity;
-	float h = p.h;
-
-	float linearDamping = 1.0f / ( 1.0f + h * sim.linearDamping );
-	float angularDamping = 1.0f / ( 1.0f + h * sim.angularDamping );
-	float gravityScale = sim.invMass > 0.0f ? sim.gravityScale : 0.0f;
-
-	b2Vec2 linearVelocityDelta = b2Add( b2MulSV( h * sim.invMass, sim.force ), b2MulSV( h * gravityScale, p.gravity ) );
-	float angularVelocityDelta = h * sim.invInertia * sim.torque;
-
-	v = b2MulAdd( linearVelocityDelta, linearDamping, v );
-	w = angularVelocityDelta + angularDamping * w;
-
-	state->linearVelocity = v;
-	state->angularVelocity = w;
+	ApplyVelocityStep( MakeVelocityStep( sim, p ), state->linearVelocity, state->angularVelocity );
 }
 
 // Position integration of one body: locks, speed caps, delta position and rotation
@@ -363,205 +463,487 @@ B2G_DEVI void IntegratePosition( BodyState* state, const StepParams& p )
 
 // ---------------------------------------------------------------------------------------------
 // Colored (wide-lane) contact arithmetic
+//
+// A lane holds its constraint as a ContactRow (the groups its stage loaded) and the velocities of
+// its two bodies; the impulse groups i1, i2 (normal, tangent, total normal impulse) and the rolling
+// impulse are updated in the row and stored by the caller.
+
+struct ContactRow
+{
+	float4 mass;	// invMassA, invIA, invMassB, invIB
+	float4 normal;	// x, y, friction, tangent speed
+	float4 soft;	// bias rate, mass scale, impulse scale, restitution
+	float4 rolling; // resistance, mass, impulse
+	float4 a1, m1, i1;
+	float4 a2, m2, i2;
+};
+
+enum RowGroup
+{
+	kgMass = kcInvMassA / 4,
+	kgNormal = kcNormalX / 4,
+	kgSoft = kcBiasRate / 4,
+	kgRolling = kcRollingResistance / 4,
+	kgAnchor1 = kcAnchorA1X / 4,
+	kgPoint1 = kcBaseSeparation1 / 4,
+	kgImpulse1 = kcNormalImpulse1 / 4,
+	kgAnchor2 = kcAnchorA2X / 4,
+	kgPoint2 = kcBaseSeparation2 / 4,
+	kgImpulse2 = kcNormalImpulse2 / 4,
+};
+
+enum ColorStage
+{
+	kStageWarmStart,
+	kStageSolve,
+	kStageRelax,
+	kStageRestitution,
+};
+
+// The groups a stage reads (the others stay as they are).
+template <int Stage>
+B2G_DEVI void LoadRow( const ConstraintSoA& c, int i, ContactRow& r )
+{
+	r.mass = c.f.Group( kgMass )[i];
+	r.normal = c.f.Group( kgNormal )[i];
+	if ( Stage == kStageSolve )
+	{
+		r.soft = c.f.Group( kgSoft )[i];
+	}
+	else
+	{
+		r.rolling = c.f.Group( kgRolling )[i];
+	}
+	r.a1 = c.f.Group( kgAnchor1 )[i];
+	r.i1 = c.f.Group( kgImpulse1 )[i];
+	r.a2 = c.f.Group( kgAnchor2 )[i];
+	r.i2 = c.f.Group( kgImpulse2 )[i];
+	if ( Stage != kStageWarmStart )
+	{
+		r.m1 = c.f.Group( kgPoint1 )[i];
+		r.m2 = c.f.Group( kgPoint2 )[i];
+	}
+}
+
+B2G_DEVI void StoreRowImpulses( const ConstraintSoA& c, int i, const ContactRow& r )
+{
+	c.f.Group( kgImpulse1 )[i] = r.i1;
+	c.f.Group( kgImpulse2 )[i] = r.i2;
+}
+
+struct PairVel
+{
+	float vAx, vAy, wA, vBx, vBy, wB;
+};
+
+// Velocity change of an impulse (Px, Py) at a point with anchors a.
+B2G_DEVI void ApplyRowImpulse( PairVel& v, const ContactRow& r, const float4& a, float Px, float Py )
+{
+	v.vAx = v.vAx - r.mass.x * Px;
+	v.vAy = v.vAy - r.mass.x * Py;
+	v.wA = v.wA - r.mass.y * ( a.x * Py - a.y * Px );
+	v.vBx = v.vBx + r.mass.z * Px;
+	v.vBy = v.vBy + r.mass.z * Py;
+	v.wB = v.wB + r.mass.w * ( a.z * Py - a.w * Px );
+}
+
+B2G_DEVI void WarmStartRowPoint( PairVel& v, const ContactRow& r, const float4& a, float4& imp )
+{
+	float nX = r.normal.x, nY = r.normal.y;
+	float tX = nY;
+	float tY = 0.0f - nX;
+	float Px = imp.x * nX + imp.y * tX;
+	float Py = imp.x * nY + imp.y * tY;
+	v.wA = v.wA - r.mass.y * ( a.x * Py - a.y * Px );
+	v.vAx = v.vAx - r.mass.x * Px;
+	v.vAy = v.vAy - r.mass.x * Py;
+	v.wB = v.wB + r.mass.w * ( a.z * Py - a.w * Px );
+	v.vBx = v.vBx + r.mass.z * Px;
+	v.vBy = v.vBy + r.mass.z * Py;
+	imp.z = imp.z + imp.x;
+}
+
+B2G_DEVI void WarmStartRow( ContactRow& r, PairVel& v )
+{
+	WarmStartRowPoint( v, r, r.a1, r.i1 );
+	WarmStartRowPoint( v, r, r.a2, r.i2 );
+	v.wA = v.wA - r.mass.y * r.rolling.z;
+	v.wB = v.wB + r.mass.w * r.rolling.z;
+}
+
+// The part of a normal point's solve that depends on the delta poses only, which no stage changes
+// between two position integrations.
+struct PointBias
+{
+	float bias, massScale, impulseScale;
+};
+
+struct RowBias
+{
+	PointBias p1, p2;
+};
+
+template <bool kUseBias>
+B2G_DEVI PointBias RowPointBias( const ContactRow& r, const float4& a, const float4& m, float dpX, float dpY, const float4& dA,
+								 const float4& dB, float inv_h, float contactSpeed )
+{
+	// moving anchors for the current separation
+	float rsAx = dA.z * a.x - dA.w * a.y;
+	float rsAy = dA.w * a.x + dA.z * a.y;
+	float rsBx = dB.z * a.z - dB.w * a.w;
+	float rsBy = dB.w * a.z + dB.z * a.w;
+
+	float dsx = dpX + ( rsBx - rsAx );
+	float dsy = dpY + ( rsBy - rsAy );
+	float s = ( r.normal.x * dsx + r.normal.y * dsy ) + m.x;
+
+	float biasRate = kUseBias ? r.soft.y * r.soft.x : 0.0f;
+	float massScale = kUseBias ? r.soft.y : 1.0f;
+	float impulseScale = kUseBias ? r.soft.z : 0.0f;
+
+	bool mask = s > 0.0f;
+	float specBias = s * inv_h;
+	float softBias = MaxW( biasRate * s, contactSpeed );
+	PointBias out;
+	out.bias = mask ? specBias : softBias;
+	out.massScale = mask ? 1.0f : massScale;
+	out.impulseScale = mask ? 0.0f : impulseScale;
+	return out;
+}
+
+// dA, dB: delta position (x, y) and rotation (c, s) of the two bodies.
+template <bool kUseBias>
+B2G_DEVI RowBias ComputeRowBias( const ContactRow& r, const float4& dA, const float4& dB, float inv_h, float contactSpeed )
+{
+	float dpX = dB.x - dA.x;
+	float dpY = dB.y - dA.y;
+	RowBias b;
+	b.p1 = RowPointBias<kUseBias>( r, r.a1, r.m1, dpX, dpY, dA, dB, inv_h, contactSpeed );
+	b.p2 = RowPointBias<kUseBias>( r, r.a2, r.m2, dpX, dpY, dA, dB, inv_h, contactSpeed );
+	return b;
+}
+
+B2G_DEVI void SolveRowNormal( PairVel& v, const ContactRow& r, const float4& a, const float4& m, float4& imp, const PointBias& b )
+{
+	float nX = r.normal.x, nY = r.normal.y;
+	float dvx = ( v.vBx - v.wB * a.w ) - ( v.vAx - v.wA * a.y );
+	float dvy = ( v.vBy + v.wB * a.z ) - ( v.vAy + v.wA * a.x );
+	float vn = dvx * nX + dvy * nY;
+
+	float negImpulse = m.y * ( b.massScale * vn + b.bias ) + b.impulseScale * imp.x;
+	float newImpulse = MaxW( imp.x - negImpulse, 0.0f );
+	float impulse = newImpulse - imp.x;
+	imp.x = newImpulse;
+	imp.z = imp.z + impulse;
+	ApplyRowImpulse( v, r, a, impulse * nX, impulse * nY );
+}
+
+B2G_DEVI void SolveRowFriction( PairVel& v, const ContactRow& r, const float4& a, const float4& m, float4& imp )
+{
+	float tX = r.normal.y;
+	float tY = 0.0f - r.normal.x;
+	float dvx = ( v.vBx - v.wB * a.w ) - ( v.vAx - v.wA * a.y );
+	float dvy = ( v.vBy + v.wB * a.z ) - ( v.vAy + v.wA * a.x );
+	float vt = dvx * tX + dvy * tY;
+	vt = vt - r.normal.w;
+
+	float negImpulse = m.z * vt;
+	float maxFriction = r.normal.z * imp.x;
+	float newImpulse = imp.y - negImpulse;
+	newImpulse = MaxW( 0.0f - maxFriction, MinW( newImpulse, maxFriction ) );
+	float impulse = newImpulse - imp.y;
+	imp.y = newImpulse;
+	ApplyRowImpulse( v, r, a, impulse * tX, impulse * tY );
+}
+
+// The velocity part of the solve (kUseBias) or relax stage. laneGroupRolling: any constraint of this
+// constraint's 4-lane group has rolling resistance (the wide solver tests the whole group).
+template <bool kUseBias>
+B2G_DEVI void SolveRow( ContactRow& r, PairVel& v, const RowBias& b, bool laneGroupRolling )
+{
+	float totalNormalImpulse = 0.0f;
+	SolveRowNormal( v, r, r.a1, r.m1, r.i1, b.p1 );
+	totalNormalImpulse = totalNormalImpulse + r.i1.x;
+	SolveRowNormal( v, r, r.a2, r.m2, r.i2, b.p2 );
+	totalNormalImpulse = totalNormalImpulse + r.i2.x;
+
+	if ( kUseBias == false )
+	{
+		if ( laneGroupRolling )
+		{
+			float deltaLambda = r.rolling.y * ( v.wA - v.wB );
+			float lambda = r.rolling.z;
+			float maxLambda = r.rolling.x * totalNormalImpulse;
+			float rolling = b2ClampFloat( lambda + deltaLambda, -maxLambda, maxLambda );
+			r.rolling.z = rolling;
+			deltaLambda = rolling - lambda;
+			v.wA = v.wA - r.mass.y * deltaLambda;
+			v.wB = v.wB + r.mass.w * deltaLambda;
+		}
+		SolveRowFriction( v, r, r.a1, r.m1, r.i1 );
+		SolveRowFriction( v, r, r.a2, r.m2, r.i2 );
+	}
+}
+
+B2G_DEVI PairVel ToPair( const LaneBody& bA, const LaneBody& bB )
+{
+	return PairVel{ bA.vx, bA.vy, bA.w, bB.vx, bB.vy, bB.w };
+}
+
+template <typename Bodies>
+B2G_DEVI void StorePair( const Bodies& B, int ia, int ib, LaneBody& bA, LaneBody& bB, const PairVel& v )
+{
+	bA.vx = v.vAx;
+	bA.vy = v.vAy;
+	bA.w = v.wA;
+	bB.vx = v.vBx;
+	bB.vy = v.vBy;
+	bB.w = v.wB;
+	B.Store( ia, bA );
+	B.Store( ib, bB );
+}
 
 template <typename Bodies>
 B2G_DEVI void WarmStartContact( const ConstraintSoA& c, int i, const Bodies& B )
 {
 	int ia = c.bodyA[i];
 	int ib = c.bodyB[i];
+	ContactRow r;
+	LoadRow<kStageWarmStart>( c, i, r );
 	LaneBody bA = B.Load( ia );
 	LaneBody bB = B.Load( ib );
-
-	float mA = c.f[kcInvMassA][i], mB = c.f[kcInvMassB][i];
-	float iA = c.f[kcInvIA][i], iB = c.f[kcInvIB][i];
-	float nX = c.f[kcNormalX][i], nY = c.f[kcNormalY][i];
-	float tX = nY;
-	float tY = 0.0f - nX;
-
-	{
-		float rAx = c.f[kcAnchorA1X][i], rAy = c.f[kcAnchorA1Y][i];
-		float rBx = c.f[kcAnchorB1X][i], rBy = c.f[kcAnchorB1Y][i];
-		float ni = c.f[kcNormalImpulse1][i], ti = c.f[kcTangentImpulse1][i];
-		float Px = ni * nX + ti * tX;
-		float Py = ni * nY + ti * tY;
-		bA.w = bA.w - iA * ( rAx * Py - rAy * Px );
-		bA.vx = bA.vx - mA * Px;
-		bA.vy = bA.vy - mA * Py;
-		bB.w = bB.w + iB * ( rBx * Py - rBy * Px );
-		bB.vx = bB.vx + mB * Px;
-		bB.vy = bB.vy + mB * Py;
-		c.f[kcTotalNormalImpulse1][i] = c.f[kcTotalNormalImpulse1][i] + ni;
-	}
-
-	{
-		float rAx = c.f[kcAnchorA2X][i], rAy = c.f[kcAnchorA2Y][i];
-		float rBx = c.f[kcAnchorB2X][i], rBy = c.f[kcAnchorB2Y][i];
-		float ni = c.f[kcNormalImpulse2][i], ti = c.f[kcTangentImpulse2][i];
-		float Px = ni * nX + ti * tX;
-		float Py = ni * nY + ti * tY;
-		bA.w = bA.w - iA * ( rAx * Py - rAy * Px );
-		bA.vx = bA.vx - mA * Px;
-		bA.vy = bA.vy - mA * Py;
-		bB.w = bB.w + iB * ( rBx * Py - rBy * Px );
-		bB.vx = bB.vx + mB * Px;
-		bB.vy = bB.vy + mB * Py;
-		c.f[kcTotalNormalImpulse2][i] = c.f[kcTotalNormalImpulse2][i] + ni;
-	}
-
-	float rolling = c.f[kcRollingImpulse][i];
-	bA.w = bA.w - iA * rolling;
-	bB.w = bB.w + iB * rolling;
-
-	B.Store( ia, bA );
-	B.Store( ib, bB );
+	PairVel v = ToPair( bA, bB );
+	WarmStartRow( r, v );
+	StoreRowImpulses( c, i, r );
+	StorePair( B, ia, ib, bA, bB, v );
 }
 
-// One normal point of the wide solve. Returns the new accumulated impulse for the rolling term.
-B2G_DEVI float SolveNormalPoint( const ConstraintSoA& c, int i, LaneBody& bA, LaneBody& bB, float mA, float mB, float iA,
-								 float iB, float nX, float nY, float dpX, float dpY, float biasRate, float massScale,
-								 float impulseScale, float inv_h, float contactSpeed, int fAx, int fAy, int fBx, int fBy,
-								 int fBase, int fNormalImpulse, int fTotal, int fNormalMass )
-{
-	float rAx = c.f[fAx][i], rAy = c.f[fAy][i];
-	float rBx = c.f[fBx][i], rBy = c.f[fBy][i];
-
-	// moving anchors for the current separation
-	float rsAx = bA.dqc * rAx - bA.dqs * rAy;
-	float rsAy = bA.dqs * rAx + bA.dqc * rAy;
-	float rsBx = bB.dqc * rBx - bB.dqs * rBy;
-	float rsBy = bB.dqs * rBx + bB.dqc * rBy;
-
-	float dsx = dpX + ( rsBx - rsAx );
-	float dsy = dpY + ( rsBy - rsAy );
-	float s = ( nX * dsx + nY * dsy ) + c.f[fBase][i];
-
-	bool mask = s > 0.0f;
-	float specBias = s * inv_h;
-	float softBias = MaxW( biasRate * s, contactSpeed );
-	float bias = mask ? specBias : softBias;
-	float pointMassScale = mask ? 1.0f : massScale;
-	float pointImpulseScale = mask ? 0.0f : impulseScale;
-
-	float dvx = ( bB.vx - bB.w * rBy ) - ( bA.vx - bA.w * rAy );
-	float dvy = ( bB.vy + bB.w * rBx ) - ( bA.vy + bA.w * rAx );
-	float vn = dvx * nX + dvy * nY;
-
-	float normalImpulse = c.f[fNormalImpulse][i];
-	float negImpulse = c.f[fNormalMass][i] * ( pointMassScale * vn + bias ) + pointImpulseScale * normalImpulse;
-	float newImpulse = MaxW( normalImpulse - negImpulse, 0.0f );
-	float impulse = newImpulse - normalImpulse;
-	c.f[fNormalImpulse][i] = newImpulse;
-	c.f[fTotal][i] = c.f[fTotal][i] + impulse;
-
-	float Px = impulse * nX;
-	float Py = impulse * nY;
-	bA.vx = bA.vx - mA * Px;
-	bA.vy = bA.vy - mA * Py;
-	bA.w = bA.w - iA * ( rAx * Py - rAy * Px );
-	bB.vx = bB.vx + mB * Px;
-	bB.vy = bB.vy + mB * Py;
-	bB.w = bB.w + iB * ( rBx * Py - rBy * Px );
-	return newImpulse;
-}
-
-B2G_DEVI void FrictionPoint( const ConstraintSoA& c, int i, LaneBody& bA, LaneBody& bB, float mA, float mB, float iA, float iB,
-							 float tX, float tY, float friction, float tangentSpeed, int fAx, int fAy, int fBx, int fBy,
-							 int fNormalImpulse, int fTangentImpulse, int fTangentMass )
-{
-	float rAx = c.f[fAx][i], rAy = c.f[fAy][i];
-	float rBx = c.f[fBx][i], rBy = c.f[fBy][i];
-
-	float dvx = ( bB.vx - bB.w * rBy ) - ( bA.vx - bA.w * rAy );
-	float dvy = ( bB.vy + bB.w * rBx ) - ( bA.vy + bA.w * rAx );
-	float vt = dvx * tX + dvy * tY;
-	vt = vt - tangentSpeed;
-
-	float negImpulse = c.f[fTangentMass][i] * vt;
-	float maxFriction = friction * c.f[fNormalImpulse][i];
-	float tangentImpulse = c.f[fTangentImpulse][i];
-	float newImpulse = tangentImpulse - negImpulse;
-	newImpulse = MaxW( 0.0f - maxFriction, MinW( newImpulse, maxFriction ) );
-	float impulse = newImpulse - tangentImpulse;
-	c.f[fTangentImpulse][i] = newImpulse;
-
-	float Px = impulse * tX;
-	float Py = impulse * tY;
-	bA.vx = bA.vx - mA * Px;
-	bA.vy = bA.vy - mA * Py;
-	bA.w = bA.w - iA * ( rAx * Py - rAy * Px );
-	bB.vx = bB.vx + mB * Px;
-	bB.vy = bB.vy + mB * Py;
-	bB.w = bB.w + iB * ( rBx * Py - rBy * Px );
-}
-
-// laneGroupRolling: true when any constraint of this constraint's 4-lane group has rolling
-// resistance (the wide solver tests the whole group).
-template <typename Bodies>
-B2G_DEVI void SolveContact( const ConstraintSoA& c, int i, const Bodies& B, bool useBias, float inv_h, float contactSpeed,
-							bool laneGroupRolling )
+// rolling( row ): whether the constraint's 4-lane group has rolling resistance (relax stage only).
+template <bool kUseBias, typename Bodies, typename Rolling>
+B2G_DEVI void SolveContact( const ConstraintSoA& c, int i, const Bodies& B, float inv_h, float contactSpeed, Rolling rolling )
 {
 	int ia = c.bodyA[i];
 	int ib = c.bodyB[i];
+	ContactRow r;
+	LoadRow<kUseBias ? kStageSolve : kStageRelax>( c, i, r );
 	LaneBody bA = B.Load( ia );
 	LaneBody bB = B.Load( ib );
-
-	float mA = c.f[kcInvMassA][i], mB = c.f[kcInvMassB][i];
-	float iA = c.f[kcInvIA][i], iB = c.f[kcInvIB][i];
-	float nX = c.f[kcNormalX][i], nY = c.f[kcNormalY][i];
-
-	float biasRate, massScale, impulseScale;
-	if ( useBias )
+	float4 dA = make_float4( bA.dpx, bA.dpy, bA.dqc, bA.dqs );
+	float4 dB = make_float4( bB.dpx, bB.dpy, bB.dqc, bB.dqs );
+	RowBias bias = ComputeRowBias<kUseBias>( r, dA, dB, inv_h, contactSpeed );
+	PairVel v = ToPair( bA, bB );
+	bool laneGroupRolling = kUseBias == false && rolling( r );
+	SolveRow<kUseBias>( r, v, bias, laneGroupRolling );
+	StoreRowImpulses( c, i, r );
+	if ( laneGroupRolling )
 	{
-		biasRate = c.f[kcMassScale][i] * c.f[kcBiasRate][i];
-		massScale = c.f[kcMassScale][i];
-		impulseScale = c.f[kcImpulseScale][i];
+		c.f[kcRollingImpulse][i] = r.rolling.z;
+	}
+	StorePair( B, ia, ib, bA, bB, v );
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same arithmetic with two neighbouring lanes per constraint, the even one for body A and the odd
+// one for body B: each holds its own body's velocity, anchors and masses. The terms of the relative
+// velocity are formed in both lanes at once and exchanged within the pair, and each lane applies the
+// impulse to its own body, which takes a quarter of the instructions off a constraint's serial path
+// and halves its LDS traffic. Body A's masses are negated: v - m * P and v + ( -m ) * P are the same
+// float, so every value is that of the one-lane form.
+
+// x of the pair's lane A and of its lane B (DPP quad permutations).
+B2G_DEVI float PairA( float x )
+{
+	return __uint_as_float( __builtin_amdgcn_mov_dpp( __float_as_uint( x ), 0xA0, 0xF, 0xF, true ) ); // 0, 0, 2, 2
+}
+
+B2G_DEVI float PairB( float x )
+{
+	return __uint_as_float( __builtin_amdgcn_mov_dpp( __float_as_uint( x ), 0xF5, 0xF, 0xF, true ) ); // 1, 1, 3, 3
+}
+
+// Native vectors: a row in flight is one register tuple per load.
+typedef float F2 __attribute__( ( ext_vector_type( 2 ) ) );
+typedef float F4 __attribute__( ( ext_vector_type( 4 ) ) );
+
+B2G_DEVI F4 PairGroup( const ConstraintSoA& c, int group, int i )
+{
+	return reinterpret_cast<const F4*>( c.f.Group( group ) )[i];
+}
+
+struct PairRow
+{
+	F2 mass;	// own inverse mass and inertia, negated for body A
+	F4 normal;	// x, y, friction, tangent speed
+	F4 soft;	// bias rate, mass scale, impulse scale, -
+	F4 rolling; // resistance, mass, impulse, -
+	F2 a1, a2;	// own anchors
+	F4 m1, m2;	// base separation, normal mass, tangent mass, -
+	F4 i1, i2;	// normal, tangent, total normal impulse, -
+};
+
+// The groups a stage reads (the others stay as they are).
+template <int Stage>
+B2G_DEVI void LoadPairRow( const ConstraintSoA& c, int i, int side, PairRow& r )
+{
+	r.mass = reinterpret_cast<const F2*>( c.f.Group( kgMass ) + i )[side];
+	r.normal = PairGroup( c, kgNormal, i );
+	if ( Stage == kStageSolve )
+	{
+		r.soft = PairGroup( c, kgSoft, i );
 	}
 	else
 	{
-		biasRate = 0.0f;
-		massScale = 1.0f;
-		impulseScale = 0.0f;
+		r.rolling = PairGroup( c, kgRolling, i );
 	}
+	r.a1 = reinterpret_cast<const F2*>( c.f.Group( kgAnchor1 ) + i )[side];
+	r.i1 = PairGroup( c, kgImpulse1, i );
+	r.a2 = reinterpret_cast<const F2*>( c.f.Group( kgAnchor2 ) + i )[side];
+	r.i2 = PairGroup( c, kgImpulse2, i );
+	if ( Stage != kStageWarmStart )
+	{
+		r.m1 = PairGroup( c, kgPoint1, i );
+		r.m2 = PairGroup( c, kgPoint2, i );
+	}
+}
 
-	float dpX = bB.dpx - bA.dpx;
-	float dpY = bB.dpy - bA.dpy;
+// Lane A stores point 1's impulses, lane B point 2's.
+B2G_DEVI void StorePairImpulses( const ConstraintSoA& c, int i, int side, const PairRow& r )
+{
+	F4 impulse;
+	impulse.x = side == 0 ? r.i1.x : r.i2.x;
+	impulse.y = side == 0 ? r.i1.y : r.i2.y;
+	impulse.z = side == 0 ? r.i1.z : r.i2.z;
+	impulse.w = 0.0f;
+	reinterpret_cast<F4*>( c.f.Group( side == 0 ? kgImpulse1 : kgImpulse2 ) )[i] = impulse;
+}
 
+struct OwnVel
+{
+	float x, y, w;
+};
+
+B2G_DEVI void ApplyPairImpulse( OwnVel& v, F2 mass, F2 a, float Px, float Py )
+{
+	v.x = v.x + mass.x * Px;
+	v.y = v.y + mass.x * Py;
+	v.w = v.w + mass.y * ( a.x * Py - a.y * Px );
+}
+
+B2G_DEVI void WarmStartPairPoint( OwnVel& v, const PairRow& r, F2 mass, F2 a, F4& imp )
+{
+	float nX = r.normal.x, nY = r.normal.y;
+	float tX = nY;
+	float tY = 0.0f - nX;
+	float Px = imp.x * nX + imp.y * tX;
+	float Py = imp.x * nY + imp.y * tY;
+	ApplyPairImpulse( v, mass, a, Px, Py );
+	imp.z = imp.z + imp.x;
+}
+
+B2G_DEVI void WarmStartPair( PairRow& r, F2 mass, OwnVel& v )
+{
+	WarmStartPairPoint( v, r, mass, r.a1, r.i1 );
+	WarmStartPairPoint( v, r, mass, r.a2, r.i2 );
+	v.w = v.w + mass.y * r.rolling.z;
+}
+
+// d: own delta position (x, y) and rotation (c, s).
+template <bool kUseBias>
+B2G_DEVI PointBias PairPointBias( const PairRow& r, F2 a, const F4& m, float dpX, float dpY, const F4& d, float inv_h,
+								  float contactSpeed )
+{
+	float rsx = d.z * a.x - d.w * a.y;
+	float rsy = d.w * a.x + d.z * a.y;
+	float dsx = dpX + ( PairB( rsx ) - PairA( rsx ) );
+	float dsy = dpY + ( PairB( rsy ) - PairA( rsy ) );
+	float s = ( r.normal.x * dsx + r.normal.y * dsy ) + m.x;
+
+	float biasRate = kUseBias ? r.soft.y * r.soft.x : 0.0f;
+	bool mask = s > 0.0f;
+	float specBias = s * inv_h;
+	float softBias = MaxW( biasRate * s, contactSpeed );
+	PointBias out;
+	out.bias = mask ? specBias : softBias;
+	out.massScale = kUseBias == false || mask ? 1.0f : r.soft.y;
+	out.impulseScale = kUseBias == false || mask ? 0.0f : r.soft.z;
+	return out;
+}
+
+template <bool kUseBias>
+B2G_DEVI RowBias ComputePairBias( const PairRow& r, const F4& d, float inv_h, float contactSpeed )
+{
+	float dpX = PairB( d.x ) - PairA( d.x );
+	float dpY = PairB( d.y ) - PairA( d.y );
+	RowBias b;
+	b.p1 = PairPointBias<kUseBias>( r, r.a1, r.m1, dpX, dpY, d, inv_h, contactSpeed );
+	b.p2 = PairPointBias<kUseBias>( r, r.a2, r.m2, dpX, dpY, d, inv_h, contactSpeed );
+	return b;
+}
+
+// Relative velocity of the two bodies at a point along (x, y).
+B2G_DEVI float PairRelativeVelocity( const OwnVel& v, F2 a, float x, float y )
+{
+	float px = v.x - v.w * a.y;
+	float py = v.y + v.w * a.x;
+	float dvx = PairB( px ) - PairA( px );
+	float dvy = PairB( py ) - PairA( py );
+	return dvx * x + dvy * y;
+}
+
+template <bool kUseBias>
+B2G_DEVI void SolvePairNormal( OwnVel& v, const PairRow& r, F2 mass, F2 a, const F4& m, F4& imp, const PointBias& b )
+{
+	float nX = r.normal.x, nY = r.normal.y;
+	float vn = PairRelativeVelocity( v, a, nX, nY );
+	// without the bias the scales are 1 and 0 (impulses are finite, so 0 * impulse adds +0)
+	float negImpulse = m.y * ( b.massScale * vn + b.bias ) + b.impulseScale * imp.x;
+	float newImpulse = MaxW( imp.x - negImpulse, 0.0f );
+	float impulse = newImpulse - imp.x;
+	imp.x = newImpulse;
+	imp.z = imp.z + impulse;
+	ApplyPairImpulse( v, mass, a, impulse * nX, impulse * nY );
+}
+
+B2G_DEVI void SolvePairFriction( OwnVel& v, const PairRow& r, F2 mass, F2 a, const F4& m, F4& imp )
+{
+	float tX = r.normal.y;
+	float tY = 0.0f - r.normal.x;
+	float vt = PairRelativeVelocity( v, a, tX, tY );
+	vt = vt - r.normal.w;
+
+	float negImpulse = m.z * vt;
+	float maxFriction = r.normal.z * imp.x;
+	float newImpulse = imp.y - negImpulse;
+	newImpulse = MaxW( 0.0f - maxFriction, MinW( newImpulse, maxFriction ) );
+	float impulse = newImpulse - imp.y;
+	imp.y = newImpulse;
+	ApplyPairImpulse( v, mass, a, impulse * tX, impulse * tY );
+}
+
+template <bool kUseBias>
+B2G_DEVI void SolvePair( PairRow& r, F2 mass, OwnVel& v, const RowBias& b, bool laneGroupRolling )
+{
 	float totalNormalImpulse = 0.0f;
-	float n1 = SolveNormalPoint( c, i, bA, bB, mA, mB, iA, iB, nX, nY, dpX, dpY, biasRate, massScale, impulseScale, inv_h,
-								 contactSpeed, kcAnchorA1X, kcAnchorA1Y, kcAnchorB1X, kcAnchorB1Y, kcBaseSeparation1,
-								 kcNormalImpulse1, kcTotalNormalImpulse1, kcNormalMass1 );
-	totalNormalImpulse = totalNormalImpulse + n1;
-	float n2 = SolveNormalPoint( c, i, bA, bB, mA, mB, iA, iB, nX, nY, dpX, dpY, biasRate, massScale, impulseScale, inv_h,
-								 contactSpeed, kcAnchorA2X, kcAnchorA2Y, kcAnchorB2X, kcAnchorB2Y, kcBaseSeparation2,
-								 kcNormalImpulse2, kcTotalNormalImpulse2, kcNormalMass2 );
-	totalNormalImpulse = totalNormalImpulse + n2;
+	SolvePairNormal<kUseBias>( v, r, mass, r.a1, r.m1, r.i1, b.p1 );
+	totalNormalImpulse = totalNormalImpulse + r.i1.x;
+	SolvePairNormal<kUseBias>( v, r, mass, r.a2, r.m2, r.i2, b.p2 );
+	totalNormalImpulse = totalNormalImpulse + r.i2.x;
 
-	if ( useBias == false )
+	if ( kUseBias == false )
 	{
 		if ( laneGroupRolling )
 		{
-			float deltaLambda = c.f[kcRollingMass][i] * ( bA.w - bB.w );
-			float lambda = c.f[kcRollingImpulse][i];
-			float maxLambda = c.f[kcRollingResistance][i] * totalNormalImpulse;
+			float deltaLambda = r.rolling.y * ( PairA( v.w ) - PairB( v.w ) );
+			float lambda = r.rolling.z;
+			float maxLambda = r.rolling.x * totalNormalImpulse;
 			float rolling = b2ClampFloat( lambda + deltaLambda, -maxLambda, maxLambda );
-			c.f[kcRollingImpulse][i] = rolling;
+			r.rolling.z = rolling;
 			deltaLambda = rolling - lambda;
-			bA.w = bA.w - iA * deltaLambda;
-			bB.w = bB.w + iB * deltaLambda;
+			v.w = v.w + mass.y * deltaLambda;
 		}
-
-		float tX = nY;
-		float tY = 0.0f - nX;
-		float friction = c.f[kcFriction][i];
-		float tangentSpeed = c.f[kcTangentSpeed][i];
-		FrictionPoint( c, i, bA, bB, mA, mB, iA, iB, tX, tY, friction, tangentSpeed, kcAnchorA1X, kcAnchorA1Y, kcAnchorB1X,
-					   kcAnchorB1Y, kcNormalImpulse1, kcTangentImpulse1, kcTangentMass1 );
-		FrictionPoint( c, i, bA, bB, mA, mB, iA, iB, tX, tY, friction, tangentSpeed, kcAnchorA2X, kcAnchorA2Y, kcAnchorB2X,
-					   kcAnchorB2Y, kcNormalImpulse2, kcTangentImpulse2, kcTangentMass2 );
+		SolvePairFriction( v, r, mass, r.a1, r.m1, r.i1 );
+		SolvePairFriction( v, r, mass, r.a2, r.m2, r.i2 );
 	}
-
-	B.Store( ia, bA );
-	B.Store( ib, bB );
 }
 
 B2G_DEVI void RestitutionPoint( const ConstraintSoA& c, int i, LaneBody& bA, LaneBody& bB, float mA, float mB, float iA,

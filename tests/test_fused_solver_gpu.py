@@ -1,0 +1,81 @@
+"""The single-workgroup solver's forms (rows resident in registers, rows streamed, general) against the
+color kernels, bit for bit after every step, at the sizes where a form's chunks change: one chunk per
+color, partial chunks, the last resident world and the first streamed one, several chunks of one color
+in a wavefront."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import box2d_amd
+from box2d_amd import WorldId
+from b2types import c_float
+
+pytestmark = pytest.mark.gpu
+
+
+class Id(ctypes.Structure):
+    _fields_ = [("index1", ctypes.c_int32), ("world0", ctypes.c_uint16), ("generation", ctypes.c_uint16)]
+
+
+class Material(ctypes.Structure):
+    _fields_ = [("friction", c_float), ("restitution", c_float), ("rollingResistance", c_float), ("tangentSpeed", c_float),
+                ("userMaterialId", ctypes.c_uint64), ("customColor", ctypes.c_uint32)]
+
+
+class BodyEvents(ctypes.Structure):
+    _fields_ = [("moveEvents", ctypes.c_void_p), ("moveCount", ctypes.c_int)]
+
+
+def _set_materials(lib, world, restitution):
+    """Every third moving body's shape gets rolling resistance and tangent speed (and restitution)."""
+    lib.b2World_GetBodyEvents.restype, lib.b2World_GetBodyEvents.argtypes = BodyEvents, [WorldId]
+    lib.b2Body_GetShapes.argtypes = [Id, ctypes.POINTER(Id), ctypes.c_int]
+    lib.b2Shape_SetSurfaceMaterial.argtypes = [Id, ctypes.POINTER(Material)]
+    events = lib.b2World_GetBodyEvents(world)
+    raw = np.frombuffer(ctypes.string_at(events.moveEvents, 40 * events.moveCount), dtype=np.uint8).reshape(-1, 40)
+    for body in sorted(raw[:, 24:32].tolist())[::3]:
+        shapes = (Id * 4)()
+        for k in range(lib.b2Body_GetShapes(Id.from_buffer_copy(bytes(body)), shapes, 4)):
+            m = Material(0.5, 0.4 if restitution else 0.0, 0.15, 0.3, 0, 0)
+            lib.b2Shape_SetSurfaceMaterial(shapes[k], ctypes.byref(m))
+
+
+def _run(scenes, make, path, steps, materials):
+    lib = box2d_amd.library()
+    h = make()
+    try:
+        world = scenes.world_id(h)
+        box2d_amd.set_solver_path(world, path)
+        scenes.step(h, 1)
+        if materials is not None:
+            _set_materials(lib, world, materials == "bouncy")
+        out = []
+        for _ in range(steps):
+            scenes.step(h, 1)
+            out.append((scenes.transforms(h).tobytes(), scenes.velocities(h).tobytes()))
+        return out, scenes.counters(h)["awake_contacts"]
+    finally:
+        scenes.destroy(h)
+
+
+CASES = [("pyramid", rows, None, 40) for rows in (1, 2, 7, 11, 16, 21, 22, 23, 24, 25, 40)]
+CASES += [("pile", n, m, 150) for n in (1, 3, 33, 130) for m in (None, "rolling", "bouncy")]
+CASES += [("pile", 600, "rolling", 200), ("chains", 160, None, 40)]
+
+
+@pytest.mark.parametrize("kind,size,materials,steps", CASES)
+def test_fused_matches_color_kernels(gpu_scenes, kind, size, materials, steps):
+    def make():
+        if kind == "pyramid":
+            return gpu_scenes.pyramid(size)
+        if kind == "pile":
+            return gpu_scenes.create(box2d_amd.SCENE_MIXED_PILE, (size, 0, 77))
+        return gpu_scenes.create(box2d_amd.SCENE_BATCH_WORLD, (size, 2, 5))
+
+    fused, contacts = _run(gpu_scenes, make, box2d_amd.SOLVER_FUSED, steps, materials)
+    colored, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
+    assert kind == "chains" or contacts > 0
+    for k, (a, b) in enumerate(zip(fused, colored)):
+        assert a == b, f"step {k + 2}"
