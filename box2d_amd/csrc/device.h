@@ -29,6 +29,7 @@ struct SolverLists
 	int overflowContactCount = 0;
 	int overflowJointStart = 0;
 	int overflowJointCount = 0;
+	bool awakeKinematic = false; // an awake body is kinematic
 
 	// Warm start by body: for awake index i, entries [warmStart[i], warmStart[i + 1]) of warmList
 	// are the body's constraints in the warm-start stage's order (overflow joints, overflow
@@ -210,7 +211,7 @@ public:
 	void SetSolverPath( int path );
 	// Whether the next solve of a world with these list sizes takes the color-kernel path with the
 	// warm start body by body (the host then builds the per-body warm-start lists).
-	bool WantsWarmLists( int bodyCount, int constraintCount, int activeColorCount, int overflowCount ) const;
+	bool WantsWarmLists( const SolverLists& lists ) const;
 
 	// Step recording for the adjoint: while a tape is set, every solve appends one record (body
 	// state at the step's start, constraints in solve order) to the tape. index is the world's

@@ -416,7 +416,29 @@ struct PrepareArgs
 	const BodyAux* aux;
 	const int* bodySlot;
 	StepParams p;
+	// XCD solver (else null): per slot the colors of the body's constraints
+	unsigned int* masks;
+	int colors;
+	int colorStart[25];
 };
+
+// The color bit of list position i, into the masks of its two bodies.
+B2G_DEV void MarkColor( unsigned int* masks, const int* colorStart, int colors, int i, int slotA, int slotB )
+{
+	int color = 0;
+	while ( color + 1 < colors && i >= colorStart[color + 1] )
+	{
+		color += 1;
+	}
+	if ( slotA != kStaticSlot )
+	{
+		atomicOr( masks + slotA, 1u << color );
+	}
+	if ( slotB != kStaticSlot )
+	{
+		atomicOr( masks + slotB, 1u << color );
+	}
+}
 
 // Constraint preparation (reference src/contact_solver.c:1573-1809; the overflow variant at
 // :24-160 computes the same values).
@@ -439,8 +461,14 @@ B2G_DEV void PrepareContactsBody( const PrepareArgs& a, int i )
 
 	bool staticA = a.aux[bodyIdA].type == b2_staticBody;
 	bool staticB = a.aux[bodyIdB].type == b2_staticBody;
-	c.slotA[i] = staticA ? kStaticSlot : a.bodySlot[bodyIdA];
-	c.slotB[i] = staticB ? kStaticSlot : a.bodySlot[bodyIdB];
+	const int slotA = staticA ? kStaticSlot : a.bodySlot[bodyIdA];
+	const int slotB = staticB ? kStaticSlot : a.bodySlot[bodyIdB];
+	c.slotA[i] = slotA;
+	c.slotB[i] = slotB;
+	if ( a.masks != nullptr )
+	{
+		MarkColor( a.masks, a.colorStart, a.colors, i, slotA, slotB );
+	}
 
 	float mA = a.sims[bodyIdA].invMass;
 	float iA = a.sims[bodyIdA].invInertia;
@@ -530,6 +558,10 @@ struct PrepareJointArgs
 	const BodyAux* aux;
 	const int* bodySlot;
 	StepParams p;
+	// as in PrepareArgs
+	unsigned int* masks;
+	int colors;
+	int colorStart[25];
 };
 
 // Joint preparation (reference src/joint.c:1406-1452, src/revolute_joint.c:217-281).
@@ -560,6 +592,10 @@ B2G_DEV void PrepareJointsBody( const PrepareJointArgs& a, int k )
 	joint->indexB = joint->bodyIdB;
 	joint->slotA = a.aux[joint->bodyIdA].type == b2_staticBody ? kStaticSlot : a.bodySlot[joint->bodyIdA];
 	joint->slotB = a.aux[joint->bodyIdB].type == b2_staticBody ? kStaticSlot : a.bodySlot[joint->bodyIdB];
+	if ( a.masks != nullptr )
+	{
+		MarkColor( a.masks, a.colorStart, a.colors, k, joint->slotA, joint->slotB );
+	}
 
 	// Type terms (src/revolute_joint.c:217-281, src/weld_joint.c:148-220, src/prismatic_joint.c:295-350,
 	// src/wheel_joint.c:197-282, src/distance_joint.c:250-313, src/motor_joint.c:179-245,
@@ -1806,19 +1842,26 @@ __global__ __launch_bounds__( kForm == kFusedGeneral ? kFusedGeneralThreads : kF
 	FusedBody<kForm>( a, s_lds );
 }
 
+// Chunks of one stage: contacts by kChunk, joints by wavefronts.
+template <typename Starts>
+static int StageChunks( const Starts& contactStart, const Starts& jointStart, int colors )
+{
+	int chunks = 0;
+	for ( int c = 0; c < colors; ++c )
+	{
+		chunks += ( contactStart[c + 1] - contactStart[c] + kChunk - 1 ) / kChunk + ( jointStart[c + 1] - jointStart[c] + 63 ) / 64;
+	}
+	return chunks;
+}
+
+constexpr int kFusedResidentChunks = kResidentRows * kFusedThreads / 64;
+
 // Form and threads of a single world's fused solve: a wavefront per chunk of a stage's constraints, up
 // to the form's limit; resident when all chunks fit.
 static FusedForm FusedPlan( const FusedArgs& a, int* threads )
 {
-	int chunks = 0;
-	for ( int c = 0; c < a.activeColorCount; ++c )
-	{
-		chunks += ( a.colorContactStart[c + 1] - a.colorContactStart[c] + kChunk - 1 ) / kChunk +
-				  ( a.colorJointStart[c + 1] - a.colorJointStart[c] + 63 ) / 64;
-	}
-	const FusedForm form = FusedIsGeneral( a ) ? kFusedGeneral
-						   : chunks <= kResidentRows * kFusedThreads / 64 ? kFusedResident
-																		  : kFusedStreamed;
+	const int chunks = StageChunks( a.colorContactStart, a.colorJointStart, a.activeColorCount );
+	const FusedForm form = FusedIsGeneral( a ) ? kFusedGeneral : chunks <= kFusedResidentChunks ? kFusedResident : kFusedStreamed;
 	const int most = form == kFusedGeneral ? kFusedGeneralThreads : kFusedThreads;
 	*threads = 64;
 	while ( *threads < most && *threads < 64 * chunks )
@@ -1864,44 +1907,71 @@ __global__ __launch_bounds__( kThreads ) void SolveFusedBatchKernel( const Fused
 }
 
 // ---------------------------------------------------------------------------------------------
-// XCD solver: the whole substep loop of one world in one launch, on the compute units of one XCD.
+// XCD solver: the whole substep loop of one world in one launch, on the compute units of one XCD,
+// ordered by data instead of by barriers or kernel boundaries.
 //
-// A stage's colors are Gauss-Seidel phases, and in the color-kernel path each phase is a kernel
-// launch with a floor of 3-5 us. Here the phases are separated by a barrier among the workgroups
-// of one XCD instead. The CUs of an XCD share one L2, so a barrier only has to make each
-// workgroup's stores reach that L2 before it arrives (a wait for its outstanding memory
-// operations) and count arrivals with L2 atomics: about 1.2-1.4 us per barrier on MI355X, where
-// coherence across XCDs would mean writing back each L2 at every barrier. The launch places
-// workgroup b on XCD b mod 8 (round robin), so the grid is 8 x kXcdGroups workgroups
-// (cooperative: all resident at once); the workgroups that read XCC_ID 0 take tickets and solve,
-// the others exit at once. Every wait is bounded: a barrier that is not complete after
-// kXcdSpinLimit polls (or sees another workgroup's timeout) raises the error flag and the
-// workgroup exits, and the host stops with an error.
+// What bounds a large world's substep loop is the length of its chain of color phases (29 per
+// substep on the large pyramid), and a phase costs 3-5 us as a kernel launch and 3.5-4.5 us with a
+// barrier among workgroups. Here a constraint waits for its own two bodies only. Every awake body has
+// a record of 8-byte words in device memory, each a float and a tag; the tag counts the operations
+// applied to the body since the step began. A constraint's place in that count is known beforehand
+// (the body's constraints in color order, FlowSides), so its lane polls the body's three velocity
+// words until all carry the tag of the operation before its own, solves, and stores the new velocity
+// with the next tag. A body is written by exactly the lane whose turn it is, so the words need no
+// other order: each is valid by its own tag, whichever of them becomes visible first. Velocity integration and
+// position integration are operations of the body's own lane; the latter also publishes the delta
+// pose, tagged with the number of integrations, which is not overwritten before every constraint of
+// the body has taken its turn.
 //
-// What workgroups share must not be read from a CU's L1, which may still hold a line another CU
-// has since rewritten (measured on MI355X: plain loads read stale data, and an L1 invalidate
-// costs about 0.9 us per workgroup per barrier because it also walks the L2). Body states, the
-// only mutable data the phases exchange, are therefore read with agent-scope loads
-// (CoherentBodies), which skip the L1. Constraint and joint rows are otherwise only touched by the
-// wave that owns them: a phase's lanes are cut into 64-lane waves and wave w goes to participant
-// w mod kXcdGroups. The per-body warm start (worlds without joints) is the exception: it reads
-// other waves' impulses with the same kind of loads and leaves the total-normal-impulse sums to
-// each contact's own solve lane (AddWarmTotals); worlds with joints warm start color by color.
-// Each phase runs exactly the lanes one color kernel launch runs, in any order within the phase.
+// Constraints are taken as in the fused solver: two lanes each, in chunks of 32, chunk k of a stage to
+// wavefront k mod W, every wavefront in the order of the phases; the first kRows chunks of a
+// wavefront keep their rows in registers, the others load theirs ahead. The lowest unfinished chunk
+// never waits for a later one, so the loop ends as long as every wavefront that owns work is
+// running. That is made sure of without any assumption about the launch: the workgroups that find
+// themselves on XCD 0 register, the first of them closes the register when all that the round-robin
+// placement gives have come (or after a bounded wait), and the work is divided among those
+// registered; the others leave. Every wait is bounded: after kFlowPollLimit polls a wavefront raises
+// the error flag and ends, and the host stops with an error.
+//
+// One XCD, because its 32 CUs share an L2: a store passes the L1 to it and a load that passes the L1
+// reads it, so words travel between them in well under a microsecond, where another XCD's would pass
+// memory (the same loop with agent-scope stores, which do, took 1095 us per step on the 100-row
+// pyramid). The kernel makes sure of it by the XCC_ID register. What bounds a phase then is the way of
+// a velocity through the L2 and, per CU, the cache lines of a poll's gather: 0.6 us at the 20-row
+// pyramid, 0.75 at 100 rows. Measured per step: 100-row pyramid 279 -> 88 us, 20,000-body rain 689 ->
+// 288 us, against the color kernels; 1000-body rain 200 -> 92 us against the streamed fused solver.
+// Worlds with awake kinematic bodies (whose velocity changes with no constraint's turn) and with
+// overflow constraints go to the other solvers.
 
-constexpr int kXcdThreads = 1024;
-constexpr int kXcdGroups = 32; // workgroups on the solving XCD (one per CU of an MI355X XCD)
 constexpr int kXcdCount = 8;
-constexpr int kXcdGrid = kXcdGroups * kXcdCount;
-constexpr int kXcdWaves = kXcdThreads / 64;
-constexpr long long kXcdSpinLimit = 1 << 22; // polls before a barrier gives up (~seconds)
+constexpr int kFlowGroups = 32; // workgroups on the solving XCD (one per CU of an MI355X XCD)
+constexpr int kFlowGrid = kFlowGroups * kXcdCount;
+constexpr int kFlowClosed = 1 << 20;		  // added to the register when it closes
+constexpr int kFlowRegisterPolls = 256;		  // for the last workgroups to come
+constexpr int kFlowPollLimit = 1 << 20; // polls before a wait gives up (about a second)
+constexpr int kFlowWords = 8;				  // 8-byte words per body: velocity (3), spare, delta pose (4)
+constexpr int kFlowBodyChunks = 2;			  // body chunks of a wavefront kept in registers
 
-// sync[]: 0 ticket, 1 barrier arrivals, 2 error (barrier timeout), 3 unused
-struct XcdArgs
+// sync[]: 0 register, 1 workgroups registered, 2 error (a wait timed out); cleared by the pack
+struct FlowArgs
 {
-	FusedArgs f; // color ranges, warm lists and parameters; f.color.c holds body ids
+	ConstraintSoA c; // bodyA/B hold slots
+	JointSim* joints;
+	const int* jointList;
+	const int* awake;
+	int bodyCount;
+	const BodySim* sims;
+	BodyState* states;
+	int colors;
+	int contactStart[kMaxColorSlots + 1];
+	int jointStart[kMaxColorSlots + 1];
+	int subStepCount;
+	StepParams p;
+	unsigned long long* words; // the bodies' records, kFlowWords per slot
+	unsigned int* masks;	   // colors of a slot's constraints (from the preparation), cleared at the end
+	unsigned int* sides;	   // FlowSides per constraint and side
+	unsigned int base;		   // tags of this step start here
 	int* sync;
-	int zero; // 0, passed at run time so the barrier's polling atomic is not folded into a load
 };
 
 __device__ __forceinline__ int XccId()
@@ -1910,176 +1980,690 @@ __device__ __forceinline__ int XccId()
 	return __builtin_amdgcn_s_getreg( 20 | ( 0 << 6 ) | ( 3 << 11 ) ) & 0xF;
 }
 
-__device__ __forceinline__ int L2Poll( int* p, int zero )
+typedef unsigned int U2 __attribute__( ( ext_vector_type( 2 ) ) );
+typedef unsigned int U4 __attribute__( ( ext_vector_type( 4 ) ) );
+
+// The bodies' records: 32 bytes of velocity words per slot, then (from `pose` bytes on) 32 bytes of
+// delta-pose words per slot. Words are read 16 bytes at a time where two are neighbours (a wavefront's
+// gather costs its CU a cycle per cache line and instruction, which is what bounds a poll), with loads
+// that pass the L1; the stores go through the L1 to the L2 that the XCD's CUs share.
+struct FlowRecords
 {
-	return __hip_atomic_fetch_add( p, zero, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
+	__amdgpu_buffer_rsrc_t buffer;
+	unsigned int pose;
+};
+
+constexpr int kFlowRecordBytes = 32;
+constexpr int kFlowPassL1 = 0x10; // sc1
+
+B2G_DEV FlowRecords MakeFlowRecords( void* base, int slots )
+{
+	return FlowRecords{ __builtin_amdgcn_make_buffer_rsrc( base, 0, 2 * kFlowRecordBytes * slots, 0x00027000 ),
+						(unsigned int)( kFlowRecordBytes * slots ) };
 }
 
-// Barrier among the participants; returns false when it timed out (or another one did).
-__device__ bool XcdBarrier( const XcdArgs& a, int& arrivals )
+B2G_DEV U4 FlowLoad4( const FlowRecords& f, unsigned int offset )
 {
-	__shared__ int s_ok;
-	arrivals += kXcdGroups;
-	__builtin_amdgcn_s_waitcnt( 0 ); // this wave's stores are in L2
-	__syncthreads();
-	if ( threadIdx.x == 0 )
+	asm volatile( "" ::: "memory" ); // another wavefront may have written it
+	return __builtin_amdgcn_raw_buffer_load_b128( f.buffer, offset, 0, kFlowPassL1 );
+}
+
+B2G_DEV U2 FlowLoad2( const FlowRecords& f, unsigned int offset )
+{
+	return __builtin_amdgcn_raw_buffer_load_b64( f.buffer, offset, 0, kFlowPassL1 );
+}
+
+// One side of a constraint: slot | degree << 20 | rank << 25 (the body's constraints, and how many of
+// them have a lower color).
+B2G_DEV unsigned int FlowSides( unsigned int slot, unsigned int mask, int color )
+{
+	return slot | (unsigned int)__popc( mask ) << 20 | (unsigned int)__popc( mask & ( ( 1u << color ) - 1u ) ) << 25;
+}
+
+constexpr int kFlowMaxBodies = ( 1 << 20 ) - 1;
+
+// Tags of a body with `degree` constraints within one substep: 1 after velocity integration, then one
+// per constraint (warm start), one per constraint (solve), one after position integration, one per
+// constraint (relax).
+B2G_DEV unsigned int FlowSubstepTags( unsigned int degree )
+{
+	return 3 * degree + 2;
+}
+
+template <int Stage>
+B2G_DEV unsigned int FlowStageTag( unsigned int degree, unsigned int rank )
+{
+	return Stage == kStageWarmStart ? 1 + rank : Stage == kStageSolve ? 1 + degree + rank : 2 + 2 * degree + rank;
+}
+
+struct FlowLane
+{
+	ConstraintSoA c;
+	FlowRecords records;
+	int* sync;
+	int wave;
+	int waves;
+	int pair;
+	int side;
+	int colors;
+	int contactStarts;
+	int jointStarts;
+	float inv_h;
+	float contactSpeed;
+};
+
+// A wait that is not over after `polls` polls: gives up (ends this wavefront) past the limit.
+B2G_DEV void FlowPolled( int* sync, int& polls )
+{
+	++polls;
+	const bool other = ( polls & 0xFFF ) == 0 && __hip_atomic_load( sync + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) != 0;
+	if ( polls > kFlowPollLimit || other )
 	{
-		__hip_atomic_fetch_add( a.sync + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
-		int ok = 1;
-		long long polls = 0;
-		while ( L2Poll( a.sync + 1, a.zero ) < arrivals )
+		__hip_atomic_store( sync + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+		__builtin_amdgcn_endpgm();
+	}
+}
+
+// Wait until the body's velocity carries the tag (lanes with need false do not wait).
+B2G_DEV void FlowAwaitVelocity( const FlowLane& L, int slot, unsigned int tag, bool need, OwnVel& v )
+{
+	bool waiting = need;
+	int polls = 0;
+	while ( true )
+	{
+		unsigned int ahead = 0;
+		if ( waiting )
 		{
-			if ( ++polls > kXcdSpinLimit || L2Poll( a.sync + 2, a.zero ) != 0 )
+			U4 xy = FlowLoad4( L.records, kFlowRecordBytes * slot );
+			U2 w = FlowLoad2( L.records, kFlowRecordBytes * slot + 16 );
+			ahead = tag - w.y;
+			if ( xy.y == tag && xy.w == tag && w.y == tag )
 			{
-				__hip_atomic_fetch_add( a.sync + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
-				ok = 0;
-				break;
+				v = { __uint_as_float( xy.x ), __uint_as_float( xy.z ), __uint_as_float( w.x ) };
+				waiting = false;
 			}
 		}
-		s_ok = ok;
+		if ( __ballot( waiting ) == 0 )
+		{
+			return;
+		}
+		// some body's turn is two operations away or more: leave the caches to those who are next
+		if ( __ballot( waiting && ahead >= 2 ) != 0 )
+		{
+			__builtin_amdgcn_s_sleep( 8 );
+		}
+		FlowPolled( L.sync, polls );
 	}
-	__syncthreads();
-	return s_ok != 0;
 }
 
-// Lanes of one color of one stage, wave-interleaved over the participants.
-template <int Stage>
-B2G_DEV void XcdColor( const XcdArgs& a, const ColorRange& r, int rank, const CoherentBodies& B )
+B2G_DEV void FlowAwaitPose( const FlowLane& L, int slot, unsigned int tag, bool need, F4& d )
 {
-	int lanes = r.jointCount + r.contactCount;
-	int lane = threadIdx.x & 63;
-	for ( int lw = threadIdx.x >> 6;; lw += kXcdWaves )
+	bool waiting = need;
+	int polls = 0;
+	while ( true )
 	{
-		int w = lw * kXcdGroups + rank;
-		if ( w * 64 >= lanes )
+		if ( waiting )
+		{
+			U4 p = FlowLoad4( L.records, L.records.pose + kFlowRecordBytes * slot );
+			U4 q = FlowLoad4( L.records, L.records.pose + kFlowRecordBytes * slot + 16 );
+			if ( p.y == tag && p.w == tag && q.y == tag && q.w == tag )
+			{
+				d = F4{ __uint_as_float( p.x ), __uint_as_float( p.z ), __uint_as_float( q.x ), __uint_as_float( q.z ) };
+				waiting = false;
+			}
+		}
+		if ( __ballot( waiting ) == 0 )
+		{
+			return;
+		}
+		FlowPolled( L.sync, polls );
+	}
+}
+
+B2G_DEV void FlowPublishVelocity( const FlowLane& L, int slot, const OwnVel& v, unsigned int tag )
+{
+	U4 xy = { __float_as_uint( v.x ), tag, __float_as_uint( v.y ), tag };
+	U2 w = { __float_as_uint( v.w ), tag };
+	__builtin_amdgcn_raw_buffer_store_b128( xy, L.records.buffer, kFlowRecordBytes * slot, 0, 0 );
+	__builtin_amdgcn_raw_buffer_store_b64( w, L.records.buffer, kFlowRecordBytes * slot + 16, 0, 0 );
+	asm volatile( "" ::: "memory" ); // not later
+}
+
+B2G_DEV void FlowPublishPose( const FlowLane& L, int slot, const F4& d, unsigned int tag )
+{
+	U4 p = { __float_as_uint( d.x ), tag, __float_as_uint( d.y ), tag };
+	U4 q = { __float_as_uint( d.z ), tag, __float_as_uint( d.w ), tag };
+	__builtin_amdgcn_raw_buffer_store_b128( p, L.records.buffer, L.records.pose + kFlowRecordBytes * slot, 0, 0 );
+	__builtin_amdgcn_raw_buffer_store_b128( q, L.records.buffer, L.records.pose + kFlowRecordBytes * slot + 16, 0, 0 );
+	asm volatile( "" ::: "memory" );
+}
+
+// A wavefront's place in a stage's sequence of chunks (contacts of a color, then its joints).
+struct FlowCursor
+{
+	int color; // colors after the last chunk
+	int start;
+	int count;
+	int joint;
+	int chunk; // number within the stage
+	int base;  // chunks of the colors before
+};
+
+template <bool kJoints>
+B2G_DEV void FlowSeek( const FlowLane& L, FlowCursor& q )
+{
+	q.count = 0;
+	while ( q.color < L.colors )
+	{
+		int begin = __builtin_amdgcn_readlane( L.contactStarts, q.color );
+		int contacts = __builtin_amdgcn_readlane( L.contactStarts, q.color + 1 ) - begin;
+		int chunks = ( contacts + kChunk - 1 ) / kChunk;
+		int k = q.chunk - q.base;
+		if ( k < chunks )
+		{
+			q.joint = 0;
+			q.start = begin + kChunk * k;
+			q.count = Uniform( b2MinInt( kChunk, contacts - kChunk * k ) );
+			return;
+		}
+		if ( kJoints )
+		{
+			int jointBegin = __builtin_amdgcn_readlane( L.jointStarts, q.color );
+			int joints = __builtin_amdgcn_readlane( L.jointStarts, q.color + 1 ) - jointBegin;
+			int jointChunks = ( joints + 63 ) / 64;
+			if ( k - chunks < jointChunks )
+			{
+				q.joint = 1;
+				q.start = jointBegin + 64 * ( k - chunks );
+				q.count = Uniform( b2MinInt( 64, joints - 64 * ( k - chunks ) ) );
+				return;
+			}
+			chunks += jointChunks;
+		}
+		q.base = Uniform( q.base + chunks );
+		q.color = Uniform( q.color + 1 );
+	}
+}
+
+template <bool kJoints>
+B2G_DEV void FlowNext( const FlowLane& L, FlowCursor& q )
+{
+	q.chunk = Uniform( q.chunk + L.waves );
+	FlowSeek<kJoints>( L, q );
+}
+
+template <int Stage>
+B2G_DEV void FlowLoadRow( const FlowLane& L, const unsigned int* sides, const FlowCursor& q, ChunkRow& r )
+{
+	// a joint chunk, or none: any row
+	int i = q.joint != 0 || q.count == 0 ? 0 : q.start + b2MinInt( L.pair, q.count - 1 );
+	r.slot = (int)sides[2 * i + L.side];
+	LoadPairRow<Stage>( L.c, i, L.side, r.row );
+}
+
+// One stage's work on the constraint of a lane pair: wait for the own body, solve, publish.
+template <int Stage>
+B2G_DEV void FlowSolve( const FlowLane& L, PairRow& row, F2 mass, bool active, int slot, unsigned int tag, unsigned int poseTag,
+						F4& d, bool awaitPose, bool* rolling )
+{
+	const bool dynamic = active && slot != kStaticSlot;
+	RowBias bias;
+	if ( Stage != kStageWarmStart )
+	{
+		if ( awaitPose )
+		{
+			d = F4{ 0.0f, 0.0f, 1.0f, 0.0f };
+			FlowAwaitPose( L, slot, poseTag, dynamic, d );
+		}
+		bias = ComputePairBias<Stage == kStageSolve>( row, d, L.inv_h, L.contactSpeed );
+	}
+	OwnVel v = { 0.0f, 0.0f, 0.0f };
+	FlowAwaitVelocity( L, slot, tag, dynamic, v );
+	if ( Stage == kStageWarmStart )
+	{
+		WarmStartPair( row, mass, v );
+	}
+	else if ( Stage == kStageSolve )
+	{
+		SolvePair<true>( row, mass, v, bias, false );
+	}
+	else
+	{
+		// a group of four constraints is eight neighbouring lanes
+		unsigned long long any = __ballot( active && row.rolling.x != 0.0f );
+		*rolling = ( ( any >> ( threadIdx.x & 56 ) ) & 0xFF ) != 0;
+		SolvePair<false>( row, mass, v, bias, *rolling );
+	}
+	if ( dynamic )
+	{
+		FlowPublishVelocity( L, slot, v, tag + 1 );
+	}
+}
+
+// The two bodies of a joint in a lane's registers, as the joint functions' body view.
+struct FlowPair
+{
+	LaneBody* bodies;
+
+	B2G_DEVI LaneBody Load( int index ) const
+	{
+		return bodies[index];
+	}
+	B2G_DEVI void LoadDelta( int index, b2Vec2& dp, b2Rot& dq ) const
+	{
+		dp = { bodies[index].dpx, bodies[index].dpy };
+		dq = { bodies[index].dqc, bodies[index].dqs };
+	}
+	B2G_DEVI void Store( int index, const LaneBody& b ) const
+	{
+		if ( b.flags & kDynamicFlag )
+		{
+			bodies[index].vx = b.vx;
+			bodies[index].vy = b.vy;
+			bodies[index].w = b.w;
+		}
+	}
+	B2G_DEVI static int JointA( const JointSim* )
+	{
+		return 0;
+	}
+	B2G_DEVI static int JointB( const JointSim* )
+	{
+		return 1;
+	}
+};
+
+// One stage's work on a joint, one lane per joint.
+template <int Stage>
+B2G_DEV void FlowJoint( const FlowArgs& a, const FlowLane& L, const FlowCursor& q, int sub )
+{
+	const int lane = threadIdx.x & 63;
+	const bool active = lane < q.count;
+	JointSim* joint = a.joints + a.jointList[q.start + b2MinInt( lane, q.count - 1 )];
+	const int slots[2] = { joint->slotA, joint->slotB };
+	const unsigned int poseTag = a.base + sub + ( Stage == kStageRelax ? 1 : 0 );
+	unsigned int tags[2];
+	LaneBody bodies[2];
+#pragma unroll
+	for ( int k = 0; k < 2; ++k )
+	{
+		const bool dynamic = active && slots[k] != kStaticSlot;
+		const unsigned int side = FlowSides( slots[k], a.masks[slots[k]], q.color );
+		const unsigned int degree = side >> 20 & 31, rank = side >> 25;
+		tags[k] = a.base + sub * FlowSubstepTags( degree ) + FlowStageTag<Stage>( degree, rank );
+		F4 d = { 0.0f, 0.0f, 1.0f, 0.0f };
+		OwnVel v = { 0.0f, 0.0f, 0.0f };
+		FlowAwaitPose( L, slots[k], poseTag, dynamic, d );
+		FlowAwaitVelocity( L, slots[k], tags[k], dynamic, v );
+		bodies[k] = LaneBody{ v.x, v.y, v.w, dynamic ? (uint32_t)kDynamicFlag : 0u, d.x, d.y, d.z, d.w };
+	}
+	const FlowPair B{ bodies };
+	if ( active )
+	{
+		if ( Stage == kStageWarmStart )
+		{
+			WarmStartJoint( joint, B );
+		}
+		else
+		{
+			SolveJoint( joint, B, Stage == kStageSolve, a.p.h, a.p.inv_h );
+			// joint events, as in ColorLane
+			if ( Stage == kStageSolve && ( joint->forceThreshold < FLT_MAX || joint->torqueThreshold < FLT_MAX ) &&
+				 joint->eventFlag == 0 && JointReactionReached( joint, a.p.inv_h ) )
+			{
+				joint->eventFlag = 1;
+			}
+		}
+	}
+#pragma unroll
+	for ( int k = 0; k < 2; ++k )
+	{
+		if ( bodies[k].flags != 0 )
+		{
+			FlowPublishVelocity( L, slots[k], OwnVel{ bodies[k].vx, bodies[k].vy, bodies[k].w }, tags[k] + 1 );
+		}
+	}
+}
+
+// A body in its own lane.
+struct FlowBody
+{
+	bool active;
+	int slot;
+	unsigned int degree;
+	VelocityStep step;
+	LaneBody state;
+};
+
+B2G_DEV FlowBody FlowLoadBody( const FlowArgs& a, const FlowLane& L, int chunk )
+{
+	FlowBody b;
+	int i = 64 * chunk + ( threadIdx.x & 63 );
+	b.active = i < a.bodyCount;
+	i = b2MinInt( i, a.bodyCount - 1 );
+	b.slot = i + 1;
+	b.degree = (unsigned int)__popc( a.masks[b.slot] );
+	const int id = a.awake[i];
+	b.step = MakeVelocityStep( a.sims[id], a.p );
+	b.state = GlobalBodies{ a.states }.Load( id );
+	return b;
+}
+
+// Velocity integration of a substep (the first one starts from the body's state).
+B2G_DEV void FlowIntegrateVelocity( const FlowArgs& a, const FlowLane& L, FlowBody& b, int sub )
+{
+	const unsigned int tag = a.base + sub * FlowSubstepTags( b.degree );
+	OwnVel v = { b.state.vx, b.state.vy, b.state.w };
+	if ( sub > 0 )
+	{
+		FlowAwaitVelocity( L, b.slot, tag, b.active, v );
+	}
+	b2Vec2 linear = { v.x, v.y };
+	ApplyVelocityStep( b.step, linear, v.w );
+	if ( b.active )
+	{
+		if ( sub == 0 )
+		{
+			FlowPublishPose( L, b.slot, F4{ b.state.dpx, b.state.dpy, b.state.dqc, b.state.dqs }, a.base );
+		}
+		FlowPublishVelocity( L, b.slot, OwnVel{ linear.x, linear.y, v.w }, tag + 1 );
+	}
+}
+
+B2G_DEV void FlowIntegratePosition( const FlowArgs& a, const FlowLane& L, FlowBody& b, int sub )
+{
+	const unsigned int tag = a.base + sub * FlowSubstepTags( b.degree ) + 1 + 2 * b.degree;
+	OwnVel v = { 0.0f, 0.0f, 0.0f };
+	FlowAwaitVelocity( L, b.slot, tag, b.active, v );
+	b.state.vx = v.x;
+	b.state.vy = v.y;
+	b.state.w = v.w;
+	BodyState st = ToState( b.state );
+	IntegratePosition( &st, a.p );
+	b.state = ToLane( st );
+	if ( b.active )
+	{
+		FlowPublishPose( L, b.slot, F4{ b.state.dpx, b.state.dpy, b.state.dqc, b.state.dqs }, a.base + sub + 1 );
+		FlowPublishVelocity( L, b.slot, OwnVel{ b.state.vx, b.state.vy, b.state.w }, tag + 1 );
+	}
+}
+
+// The final velocity, and the whole state back to its record.
+B2G_DEV void FlowFinishBody( const FlowArgs& a, const FlowLane& L, const FlowBody& b )
+{
+	OwnVel v = { 0.0f, 0.0f, 0.0f };
+	FlowAwaitVelocity( L, b.slot, a.base + a.subStepCount * FlowSubstepTags( b.degree ), b.active, v );
+	if ( b.active )
+	{
+		float4* dst = reinterpret_cast<float4*>( a.states + a.awake[b.slot - 1] );
+		dst[0] = make_float4( v.x, v.y, v.w, __uint_as_float( b.state.flags ) );
+		dst[1] = make_float4( b.state.dpx, b.state.dpy, b.state.dqc, b.state.dqs );
+		a.masks[b.slot] = 0;
+	}
+}
+
+// The wavefront's chunks whose rows stay in registers.
+template <int kRows>
+struct FlowResident
+{
+	FlowCursor q[kRows];
+	PairRow row[kRows];
+	F2 mass[kRows];
+	int slot[kRows];
+	unsigned int degree[kRows];
+	unsigned int tag[kRows];
+	F4 pose[kRows];
+};
+
+template <int kRows, bool kJoints, int Stage, int NextStage>
+B2G_DEV void FlowStage( const FlowArgs& a, const FlowLane& L, FlowResident<kRows>& R, const FlowCursor& first, ChunkRow& r, int sub,
+						bool last )
+{
+#pragma unroll
+	for ( int k = 0; k < kRows; ++k )
+	{
+		if ( Uniform( R.q[k].count ) > 0 )
+		{
+			bool rolling = false;
+			const bool active = L.pair < R.q[k].count;
+			FlowSolve<Stage>( L, R.row[k], R.mass[k], active, R.slot[k], R.tag[k], a.base + sub + ( Stage == kStageRelax ? 1 : 0 ),
+							  R.pose[k], Stage == kStageRelax || sub == 0, &rolling );
+			// the next stage's tag
+			R.tag[k] += R.degree[k] + ( Stage == kStageWarmStart ? 0 : 1 );
+			if ( Stage == kStageRelax && last && active )
+			{
+				int i = R.q[k].start + L.pair;
+				StorePairImpulses( L.c, i, L.side, R.row[k] );
+				if ( rolling && L.side == 0 )
+				{
+					L.c.f[kcRollingImpulse][i] = R.row[k].rolling.z;
+				}
+			}
+		}
+	}
+
+	// the others, each loaded while the one before it is awaited elsewhere
+	FlowCursor q = first;
+	bool more = Uniform( q.color ) < L.colors;
+	while ( more )
+	{
+		if ( kJoints && Uniform( q.joint ) != 0 )
+		{
+			FlowJoint<Stage>( a, L, q, sub );
+		}
+		else
+		{
+			AwaitChunk<Stage>( r );
+			const unsigned int side = (unsigned int)r.slot;
+			const unsigned int degree = side >> 20 & 31, rank = side >> 25;
+			const bool active = L.pair < q.count;
+			const F2 mass = L.side == 0 ? -r.row.mass : r.row.mass;
+			bool rolling = false;
+			F4 d;
+			FlowSolve<Stage>( L, r.row, mass, active, (int)( side & kFlowMaxBodies ),
+							  a.base + sub * FlowSubstepTags( degree ) + FlowStageTag<Stage>( degree, rank ),
+							  a.base + sub + ( Stage == kStageRelax ? 1 : 0 ), d, true, &rolling );
+			if ( active )
+			{
+				int i = q.start + L.pair;
+				StorePairImpulses( L.c, i, L.side, r.row );
+				if ( rolling && L.side == 0 )
+				{
+					L.c.f[kcRollingImpulse][i] = r.row.rolling.z;
+				}
+			}
+		}
+		FlowNext<kJoints>( L, q );
+		more = Uniform( q.color ) < L.colors;
+		if ( more == false )
 		{
 			break;
 		}
-		int t = w * 64 + lane;
-		if ( Stage == kStageSolve && a.f.warmByBody && t >= r.jointCount && t < lanes )
-		{
-			AddWarmTotals( a.f.color.c, r.contactStart + t - r.jointCount );
-		}
-		ColorLane<Stage>( a.f.color, r, t, B );
+		FlowLoadRow<Stage>( L, a.sides, q, r );
 	}
-}
-
-template <int Stage>
-B2G_DEV bool XcdStage( const XcdArgs& a, int rank, const CoherentBodies& B, int& arrivals )
-{
-	for ( int color = 0; color < a.f.activeColorCount; ++color )
+	if ( Stage != kStageRelax || last == false )
 	{
-		ColorRange r;
-		r.jointStart = a.f.colorJointStart[color];
-		r.jointCount = a.f.colorJointStart[color + 1] - r.jointStart;
-		r.contactStart = a.f.colorContactStart[color];
-		r.contactCount = a.f.colorContactStart[color + 1] - r.contactStart;
-		int lanes = r.jointCount + r.contactCount;
-		if ( lanes == 0 || ( Stage == kStageRestitution && r.contactCount == 0 ) )
-		{
-			continue;
-		}
-		XcdColor<Stage>( a, r, rank, B );
-		if ( XcdBarrier( a, arrivals ) == false )
-		{
-			return false;
-		}
+		FlowLoadRow<NextStage>( L, a.sides, first, r );
 	}
-	return true;
 }
 
-__global__ __launch_bounds__( kXcdThreads ) void SolveXcdKernel( XcdArgs a )
+template <int kRows, int kThreads, bool kJoints>
+__global__ __launch_bounds__( kThreads ) void SolveFlowKernel( FlowArgs a )
 {
-	__shared__ int s_rank;
+	__shared__ int s_rank, s_groups;
 	if ( threadIdx.x == 0 )
 	{
 		int rank = -1;
+		int groups = 0;
 		if ( XccId() == 0 )
 		{
-			rank = __hip_atomic_fetch_add( a.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
+			rank = __hip_atomic_fetch_add( a.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+			if ( rank >= kFlowClosed )
+			{
+				rank = -1;
+			}
+			else if ( rank == 0 )
+			{
+				for ( int polls = 0; polls < kFlowRegisterPolls; ++polls )
+				{
+					if ( __hip_atomic_load( a.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) >= (int)gridDim.x / kXcdCount )
+					{
+						break;
+					}
+				}
+				groups = __hip_atomic_fetch_add( a.sync, kFlowClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+				__hip_atomic_store( a.sync + 1, groups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+			}
+			else
+			{
+				// the first registered workgroup is running: it always gets to closing the register
+				int polls = 0;
+				while ( ( groups = __hip_atomic_load( a.sync + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) ) == 0 )
+				{
+					if ( ++polls > kFlowPollLimit )
+					{
+						__hip_atomic_store( a.sync + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+						rank = -1;
+						break;
+					}
+				}
+			}
 		}
-		s_rank = rank < kXcdGroups ? rank : -1;
+		s_rank = rank;
+		s_groups = groups;
 	}
 	__syncthreads();
-	const int rank = s_rank;
-	if ( rank < 0 )
+	if ( s_rank < 0 )
 	{
 		return;
 	}
 
-	const FusedArgs& f = a.f;
-	const CoherentBodies B{ f.states };
-	const StepParams& p = f.color.p;
-	const int n = f.bodyCount;
+	constexpr int kWaves = kThreads / 64;
 	const int lane = threadIdx.x & 63;
-	int arrivals = 0;
+	FlowLane L;
+	L.c = a.c;
+	L.records = MakeFlowRecords( a.words, a.bodyCount + 1 );
+	L.sync = a.sync;
+	// neighbouring chunks go to different CUs
+	L.wave = Uniform( s_rank + (int)( threadIdx.x >> 6 ) * s_groups );
+	L.waves = Uniform( s_groups * kWaves );
+	L.pair = lane >> 1;
+	L.side = lane & 1;
+	L.colors = a.colors;
+	L.contactStarts = a.contactStart[b2MinInt( lane, L.colors )];
+	L.jointStarts = a.jointStart[b2MinInt( lane, L.colors )];
+	asm volatile( "" : "+v"( L.contactStarts ), "+v"( L.jointStarts ) );
+	L.inv_h = a.p.inv_h;
+	L.contactSpeed = -a.p.contactSpeed;
 
-	for ( int sub = 0; sub < f.subStepCount; ++sub )
+	// every own chunk's sides; the first chunks' rows
+	const int* slots = L.side == 0 ? a.c.bodyA : a.c.bodyB;
+	auto sidesOf = [&]( const FlowCursor& q ) {
+		int i = q.start + b2MinInt( L.pair, q.count - 1 );
+		unsigned int slot = (unsigned int)slots[i];
+		return FlowSides( slot, a.masks[slot], q.color );
+	};
+	FlowResident<kRows> R;
+	FlowCursor q;
+	q.color = 0;
+	q.start = 0;
+	q.joint = 0;
+	q.chunk = L.wave;
+	q.base = 0;
+	FlowSeek<kJoints>( L, q );
+#pragma unroll
+	for ( int k = 0; k < kRows; ++k )
 	{
-		for ( int lw = threadIdx.x >> 6;; lw += kXcdWaves )
+		// (up to the first joint chunk: the wavefront's order is the stage's)
+		R.q[k] = q;
+		R.q[k].count = q.joint != 0 ? 0 : q.count;
+		if ( Uniform( R.q[k].count ) > 0 )
 		{
-			int w = lw * kXcdGroups + rank;
-			if ( w * 64 >= n )
-			{
-				break;
-			}
-			int i = w * 64 + lane;
-			if ( i < n )
-			{
-				int id = f.awake[i];
-				BodyState st = B.LoadState( id );
-				IntegrateVelocity( f.sims[id], &st, p );
-				float vx = st.linearVelocity.x, vy = st.linearVelocity.y, wv = st.angularVelocity;
-				if ( f.warmByBody )
-				{
-					WarmStartBody<4, false, true>( f.color.c, f.color.joints, f.color.jointList, f.overflowContactStart, f.warmList,
-												   f.warmStart[i], f.warmStart[i + 1], B, st.deltaRotation, st.deltaPosition, vx, vy, wv );
-				}
-				f.states[id].linearVelocity = { vx, vy };
-				f.states[id].angularVelocity = wv;
-			}
-		}
-		if ( XcdBarrier( a, arrivals ) == false )
-		{
-			return;
-		}
-		if ( f.warmByBody == 0 && XcdStage<kStageWarmStart>( a, rank, B, arrivals ) == false )
-		{
-			return;
-		}
-		if ( XcdStage<kStageSolve>( a, rank, B, arrivals ) == false )
-		{
-			return;
-		}
-		for ( int lw = threadIdx.x >> 6;; lw += kXcdWaves )
-		{
-			int w = lw * kXcdGroups + rank;
-			if ( w * 64 >= n )
-			{
-				break;
-			}
-			int i = w * 64 + lane;
-			if ( i < n )
-			{
-				int id = f.awake[i];
-				BodyState st = B.LoadState( id );
-				IntegratePosition( &st, p );
-				f.states[id] = st;
-			}
-		}
-		if ( XcdBarrier( a, arrivals ) == false )
-		{
-			return;
-		}
-		if ( XcdStage<kStageRelax>( a, rank, B, arrivals ) == false )
-		{
-			return;
+			const int i = q.start + b2MinInt( L.pair, q.count - 1 );
+			LoadPairRow<kStageRelax>( L.c, i, L.side, R.row[k] );
+			R.row[k].soft = PairGroup( L.c, kgSoft, i );
+			const unsigned int side = sidesOf( q );
+			R.mass[k] = L.side == 0 ? -R.row[k].mass : R.row[k].mass;
+			R.slot[k] = (int)( side & kFlowMaxBodies );
+			R.degree[k] = side >> 20 & 31;
+			R.tag[k] = a.base + 1 + ( side >> 25 );
+			FlowNext<kJoints>( L, q );
 		}
 	}
-	if ( f.anyRestitution )
+	const FlowCursor first = q;
+	while ( Uniform( q.color ) < L.colors )
 	{
-		XcdStage<kStageRestitution>( a, rank, B, arrivals );
+		if ( ( kJoints == false || Uniform( q.joint ) == 0 ) && L.pair < q.count )
+		{
+			a.sides[2 * ( q.start + L.pair ) + L.side] = sidesOf( q );
+		}
+		FlowNext<kJoints>( L, q );
 	}
+	ChunkRow r;
+	FlowLoadRow<kStageWarmStart>( L, a.sides, first, r );
+
+	const int bodyChunks = ( a.bodyCount + 63 ) / 64;
+	FlowBody body[kFlowBodyChunks];
+#pragma unroll
+	for ( int k = 0; k < kFlowBodyChunks; ++k )
+	{
+		if ( L.wave + k * L.waves < bodyChunks )
+		{
+			body[k] = FlowLoadBody( a, L, L.wave + k * L.waves );
+		}
+	}
+
+	// op( body ) for each of the wavefront's body chunks; those beyond the registers (a register that
+	// closed early, a very large world) come from their records and go back to them
+	auto forBodies = [&]( auto op ) {
+#pragma unroll
+		for ( int k = 0; k < kFlowBodyChunks; ++k )
+		{
+			if ( L.wave + k * L.waves < bodyChunks )
+			{
+				op( body[k] );
+			}
+		}
+		for ( int chunk = L.wave + kFlowBodyChunks * L.waves; chunk < bodyChunks; chunk += L.waves )
+		{
+			FlowBody b = FlowLoadBody( a, L, chunk );
+			op( b );
+			if ( b.active )
+			{
+				float4* dst = reinterpret_cast<float4*>( a.states + a.awake[b.slot - 1] );
+				reinterpret_cast<float*>( dst )[3] = __uint_as_float( b.state.flags );
+				dst[1] = make_float4( b.state.dpx, b.state.dpy, b.state.dqc, b.state.dqs );
+			}
+		}
+	};
+	for ( int sub = 0; sub < a.subStepCount; ++sub )
+	{
+		const bool last = sub + 1 == a.subStepCount;
+		forBodies( [&]( FlowBody& b ) { FlowIntegrateVelocity( a, L, b, sub ); } );
+		FlowStage<kRows, kJoints, kStageWarmStart, kStageSolve>( a, L, R, first, r, sub, last );
+		FlowStage<kRows, kJoints, kStageSolve, kStageRelax>( a, L, R, first, r, sub, last );
+		forBodies( [&]( FlowBody& b ) { FlowIntegratePosition( a, L, b, sub ); } );
+		FlowStage<kRows, kJoints, kStageRelax, kStageWarmStart>( a, L, R, first, r, sub, last );
+	}
+	forBodies( [&]( FlowBody& b ) { FlowFinishBody( a, L, b ); } );
+}
+
+// The form of the XCD solver for a stage's chunks: four wavefronts per CU with four rows each in
+// registers, or eight with two and the rest streamed for worlds that need more (100-row pyramid: 88 us
+// per step against 114 with eight; 20,000-body rain: 288 with eight against 307).
+struct FlowPlan
+{
+	void ( *kernel )( FlowArgs );
+	int threads;
+};
+
+static FlowPlan PlanFlow( int chunks, bool joints )
+{
+	if ( chunks <= 4 * 4 * kFlowGroups )
+	{
+		return joints ? FlowPlan{ SolveFlowKernel<4, 256, true>, 256 } : FlowPlan{ SolveFlowKernel<4, 256, false>, 256 };
+	}
+	return joints ? FlowPlan{ SolveFlowKernel<2, 512, true>, 512 } : FlowPlan{ SolveFlowKernel<2, 512, false>, 512 };
 }
 
 struct StoreArgs
@@ -3161,7 +3745,7 @@ struct PackFinalizeArgs
 	unsigned long long* splitKey; // likewise
 	int islandWords;
 	int* keptShapeCount;	 // receives the enlarged-shape count before it is cleared (may be null)
-	const int* xcdSync;		 // XCD solver barrier words of this step (null when it did not run)
+	int* xcdSync;		 // XCD solver words of this step (null when it did not run)
 	JointSim* joints;		 // joint events: flagged joints are listed and their flags cleared
 	int jointCount;			 // 0 when no joint has a finite threshold
 	int jointEventOffset;	 // mailbox offset in ints
@@ -3282,7 +3866,15 @@ B2G_DEV void PackFinalizeBody( const PackFinalizeArgs& a )
 		{
 			*a.keptShapeCount = shapes;
 		}
-		a.mail[5] = a.xcdSync != nullptr ? a.xcdSync[2] : 0;
+		a.mail[5] = 0;
+		if ( a.xcdSync != nullptr )
+		{
+			// a wait timed out, or no workgroup found itself on the solving XCD
+			a.mail[5] = a.xcdSync[2] != 0 || a.xcdSync[1] == 0 ? 1 : 0;
+			a.xcdSync[0] = 0;
+			a.xcdSync[1] = 0;
+			a.xcdSync[2] = 0;
+		}
 		a.mail[6] = jointEvents;
 		a.counters[0] = 0;
 		a.counters[1] = 0;
@@ -3412,6 +4004,8 @@ struct DevArray
 		capacity = 0;
 	}
 };
+
+static bool XcdSolverUsable();
 
 struct DeviceWorld::Impl
 {
@@ -3580,9 +4174,47 @@ struct DeviceWorld::Impl
 	}
 
 	hipEvent_t ev[4] = {};
-	// XCD solver: barrier words (see SolveXcdKernel) and whether this device can run it
+	// XCD solver (SolveFlowKernel): its register and error words, whether this device can run it, the
+	// bodies' words and color masks, the constraints' sides and the next step's first tag
 	int* xcdSync = nullptr;
 	int xcdUsable = -1; // -1 not checked yet
+	bool XcdUsable()
+	{
+		if ( xcdUsable < 0 )
+		{
+			xcdUsable = XcdSolverUsable() ? 1 : 0;
+		}
+		return xcdUsable == 1;
+	}
+	DevArray<unsigned long long> flowWords;
+	DevArray<unsigned int> flowMasks;
+	DevArray<unsigned int> flowSides;
+	unsigned int flowTag = 1;
+
+	// Room for the XCD solver's bodies and constraints. New or wrapped tags must match nothing that is
+	// in the words, and the masks start clear.
+	void EnsureFlow( int bodies, int constraints, unsigned int tags )
+	{
+		if ( xcdSync == nullptr )
+		{
+			HIP_CHECK( hipMalloc( &xcdSync, 4 * sizeof( int ) ) );
+			HIP_CHECK( hipMemsetAsync( xcdSync, 0, 4 * sizeof( int ), stream ) );
+		}
+		const size_t slots = (size_t)bodies + 1;
+		const bool grown = kFlowWords * slots > flowWords.capacity;
+		if ( grown )
+		{
+			flowWords.Reserve( kFlowWords * slots, false, stream, 0 );
+			flowMasks.Reserve( flowWords.capacity / kFlowWords, false, stream, 0 );
+			HIP_CHECK( hipMemsetAsync( flowMasks.ptr, 0, flowMasks.capacity * sizeof( unsigned int ), stream ) );
+		}
+		if ( grown || flowTag > ~0u - tags )
+		{
+			HIP_CHECK( hipMemsetAsync( flowWords.ptr, 0, flowWords.capacity * sizeof( unsigned long long ), stream ) );
+			flowTag = 1;
+		}
+		flowSides.Reserve( 2 * (size_t)std::max( constraints, 1 ), false, stream, 0 );
+	}
 	// a recorded (batched) world too large for the batch's persistent solver: its solve is launched
 	// on its own after the batch's (LaunchDeferredSolve) and waited for in SolveFinish
 	bool solveDeferred = false;
@@ -3754,6 +4386,9 @@ DeviceWorld::~DeviceWorld()
 	{
 		(void)hipFree( impl->xcdSync );
 	}
+	impl->flowWords.Free();
+	impl->flowMasks.Free();
+	impl->flowSides.Free();
 	impl->sims.Free();
 	impl->transformIds.Free();
 	impl->transformOut.Free();
@@ -4215,7 +4850,7 @@ void DeviceWorld::UploadLists( const SolverLists& lists )
 		impl->slotStaging.assign( std::max( slots, 1 ), kStaticSlot );
 		for ( size_t k = 0; k < lists.awakeBodies.size(); ++k )
 		{
-			impl->slotStaging[lists.awakeBodies[k]] = (int)std::min<size_t>( k + 1, kFusedBodyCapacity );
+			impl->slotStaging[lists.awakeBodies[k]] = (int)k + 1;
 		}
 		impl->StageVector( impl->bodySlot, impl->slotStaging );
 	}
@@ -4745,8 +5380,8 @@ static bool BatchWarmByBody( int bodyCount )
 	return BatchTuningFor( BatchBucketOf( bodyCount ) ).warmByBody != 0;
 }
 
-// Whether the current device can run the XCD solver: an MI355X (8 XCDs of 32 CUs) with
-// cooperative launches and room for one of its workgroups on every CU.
+// Whether the current device is one that the XCD solver is laid out for: an MI355X with all of its 8
+// XCDs of 32 CUs.
 static bool XcdSolverUsable()
 {
 	if ( getenv( "B2AMD_NO_XCD_SOLVER" ) != nullptr )
@@ -4760,14 +5395,45 @@ static bool XcdSolverUsable()
 		(void)hipGetLastError();
 		return false;
 	}
-	int perCu = 0;
-	if ( hipOccupancyMaxActiveBlocksPerMultiprocessor( &perCu, SolveXcdKernel, kXcdThreads, 0 ) != hipSuccess )
+	return prop.multiProcessorCount == kFlowGrid && strncmp( prop.gcnArchName, "gfx950", 6 ) == 0;
+}
+
+// The solver of a world's step.
+enum SolverKind
+{
+	kSolverColors,
+	kSolverFused,
+	kSolverXcd,
+};
+
+// path: b2amd_SolverPath. Auto takes the fused solver while a stage's chunks fit its wavefronts (the
+// resident form: measured 48 us per step for the 20-row pyramid, 55 for 24 rows, 64 for a 400-body
+// pile, against 65, 66 and 82 in the XCD solver), above that the XCD solver where it applies (26 rows
+// 66 against 120 us, 500 bodies 85 against 167, a 40x40 joint net 151 against 254; 100 rows 88 against
+// 279 in the color kernels, 20,000 bodies 288 against 689). Worlds it does not apply to (overflow
+// constraints, awake kinematic bodies) keep the fused solver up to kFusedMaxContacts contacts, where
+// its one launch beats the color kernels' about 70, and the color kernels beyond.
+static SolverKind ChooseSolver( int path, const SolverLists& L, bool xcdUsable )
+{
+	const int nb = (int)L.awakeBodies.size();
+	const int nc = (int)L.constraintContacts.size();
+	const int overflow = L.overflowContactCount + L.overflowJointCount;
+	const bool colorsFit = L.activeColorCount <= kMaxColorSlots;
+	const bool fused = nb > 0 && nb <= kFusedBodyCapacity && colorsFit;
+	const bool xcd = xcdUsable && nb > 0 && nb <= kFlowMaxBodies && colorsFit && overflow == 0 && L.awakeKinematic == false;
+	switch ( path )
 	{
-		(void)hipGetLastError();
-		return false;
+		case 0:
+			return xcd && StageChunks( L.colorContactStart, L.colorJointStart, L.activeColorCount ) > kFusedResidentChunks ? kSolverXcd
+				   : fused && AutoFused( nc, overflow )																	   ? kSolverFused
+																														   : kSolverColors;
+		case 2:
+			return fused ? kSolverFused : kSolverColors;
+		case 3:
+			return xcd ? kSolverXcd : kSolverColors;
+		default:
+			return kSolverColors;
 	}
-	return prop.cooperativeLaunch != 0 && prop.multiProcessorCount == kXcdGrid && perCu >= 1 &&
-		   strncmp( prop.gcnArchName, "gfx950", 6 ) == 0;
 }
 
 void DeviceWorld::ArmLaunchHelper()
@@ -4832,9 +5498,27 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 		HIP_CHECK( hipEventRecord( impl->ev[2], s ) );
 	}
 
+	const bool xcdAllowed = rec == false && impl->deferredLaunched == false && impl->XcdUsable();
+	SolverKind solver = ChooseSolver( impl->solverPath, L, xcdAllowed );
+	if ( nb > 0 && ( rec || impl->tape != nullptr ) )
+	{
+		solver = kSolverFused; // one workgroup per world; what does not fit is refused below
+	}
+	if ( solver == kSolverXcd )
+	{
+		impl->EnsureFlow( nb, nc, ( 3 * kMaxColorSlots + 3 ) * (unsigned int)params.subStepCount );
+	}
+	unsigned int* flowMasks = solver == kSolverXcd ? impl->flowMasks.ptr : nullptr;
+
 	if ( nc > 0 )
 	{
-		PrepareArgs pa;
+		PrepareArgs pa = {};
+		pa.masks = flowMasks;
+		pa.colors = L.activeColorCount;
+		for ( int c = 0; flowMasks != nullptr && c <= L.activeColorCount; ++c )
+		{
+			pa.colorStart[c] = L.colorContactStart[c];
+		}
 		pa.c = impl->soa;
 		pa.count = nc;
 		pa.contacts = impl->contacts.ptr;
@@ -4858,7 +5542,13 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 
 	if ( nj > 0 )
 	{
-		PrepareJointArgs ja;
+		PrepareJointArgs ja = {};
+		ja.masks = flowMasks;
+		ja.colors = L.activeColorCount;
+		for ( int c = 0; flowMasks != nullptr && c <= L.activeColorCount; ++c )
+		{
+			ja.colorStart[c] = L.colorJointStart[c];
+		}
 		ja.joints = impl->joints.ptr;
 		ja.list = impl->jointList.ptr;
 		ja.count = nj;
@@ -5068,11 +5758,7 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 		}
 	};
 
-	// The fused solver runs on one compute unit: it wins while the per-color launch latency of the
-	// color kernels dominates, and loses once a world has enough constraints to need the whole GPU
-	// or overflow constraints that its single lane walks from device memory.
-	bool fits = nb > 0 && nb <= kFusedBodyCapacity && L.activeColorCount <= kMaxColorSlots;
-	bool fused = fits && ( impl->solverPath == 2 || ( impl->solverPath == 0 && AutoFused( nc, L.overflowContactCount + L.overflowJointCount ) ) );
+	const bool fits = nb > 0 && nb <= kFusedBodyCapacity && L.activeColorCount <= kMaxColorSlots;
 	// per-body warm-start lists exist when the host expected this path (see WantsWarmLists)
 	bool haveWarmLists = (int)L.warmStart.size() == nb + 1;
 
@@ -5083,7 +5769,6 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 			Fatal( "step recording needs the world's awake bodies in one workgroup's LDS (%d awake, at most %d)", nb,
 				   kFusedBodyCapacity );
 		}
-		fused = true;
 
 		TapeStore::WorldTape& wt = impl->tape->worlds[impl->tapeIndex];
 		char* dst = impl->tape->Alloc( TapeRecordBytes( nb, nc ) );
@@ -5140,73 +5825,45 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 		Fatal( "batched stepping needs every world's awake bodies in one workgroup's LDS (%d awake, at most %d)", nb,
 			   kFusedBodyCapacity );
 	}
-	if ( rec && nb > 0 )
-	{
-		fused = true;
-	}
-	// The XCD solver when asked for, for worlds without overflow constraints. Auto keeps the color
-	// kernels: on MI355X both spend about 3.5-4.5 us per color phase (the phases are bound by the
-	// gather-solve-scatter latency chain, not by the launch), and the XCD solver measured 0.46 vs
-	// 0.42 ms/step on the large pyramid and 1.73 vs 1.82 ms/step on the 20k-body rain.
-	bool noOverflow = L.overflowContactCount == 0 && L.overflowJointCount == 0;
-	bool xcd = fused == false && rec == false && impl->deferredLaunched == false && nb > 0 && noOverflow &&
-			   L.activeColorCount <= kMaxColorSlots && impl->solverPath == 3;
-	if ( xcd && impl->xcdUsable < 0 )
-	{
-		impl->xcdUsable = XcdSolverUsable() ? 1 : 0;
-		if ( impl->xcdUsable == 1 )
-		{
-			HIP_CHECK( hipMalloc( &impl->xcdSync, 4 * sizeof( int ) ) );
-		}
-	}
-	xcd = xcd && impl->xcdUsable == 1;
-
+	const bool xcd = solver == kSolverXcd;
 	if ( xcd )
 	{
-		XcdArgs xa;
-		FusedArgs& fa = xa.f;
-		fa.color = ca; // body ids (GlobalBodies)
-		fa.awake = impl->awakeBodies.ptr;
-		fa.bodyCount = nb;
-		fa.sims = impl->sims.ptr;
-		fa.states = impl->states.ptr;
-		fa.activeColorCount = L.activeColorCount;
+		FlowArgs xa = {};
+		xa.c = impl->soa;
+		xa.c.bodyA = impl->soa.slotA;
+		xa.c.bodyB = impl->soa.slotB;
+		xa.joints = impl->joints.ptr;
+		xa.jointList = impl->jointList.ptr;
+		xa.awake = impl->awakeBodies.ptr;
+		xa.bodyCount = nb;
+		xa.sims = impl->sims.ptr;
+		xa.states = impl->states.ptr;
+		xa.colors = L.activeColorCount;
 		for ( int c = 0; c <= L.activeColorCount; ++c )
 		{
-			fa.colorContactStart[c] = L.colorContactStart[c];
-			fa.colorJointStart[c] = L.colorJointStart[c];
+			xa.contactStart[c] = L.colorContactStart[c];
+			xa.jointStart[c] = L.colorJointStart[c];
 		}
-		fa.overflowContactStart = L.overflowContactStart;
-		fa.overflowContactCount = 0;
-		fa.overflowJointStart = L.overflowJointStart;
-		fa.overflowJointCount = 0;
-		fa.subStepCount = params.subStepCount;
-		fa.anyRestitution = anyRestitution ? 1 : 0;
-		// per body when the world has no joints (joint rows would cross workgroups)
-		fa.warmStart = impl->warmStart.ptr;
-		fa.warmList = impl->warmList.ptr;
-		fa.warmByBody = WarmByBody( false ) && haveWarmLists && nj == 0 ? 1 : 0;
+		xa.subStepCount = params.subStepCount;
+		xa.p = params;
+		xa.words = impl->flowWords.ptr;
+		xa.masks = flowMasks;
+		xa.sides = impl->flowSides.ptr;
+		xa.base = impl->flowTag;
 		xa.sync = impl->xcdSync;
-		xa.zero = 0;
+		impl->flowTag += ( 3 * kMaxColorSlots + 3 ) * (unsigned int)params.subStepCount;
 		double bytes = params.subStepCount * ( ( kBytesIntegrateVelocities + kBytesIntegratePositions ) * nb +
-											   ( kBytesWarmStart + kBytesSolve + kBytesRelax ) * nc + 3.0 * kBytesJoint * nj ) +
-					   ( anyRestitution ? kBytesRestitution * nc : 0.0 );
-		HIP_CHECK( hipMemsetAsync( impl->xcdSync, 0, 4 * sizeof( int ), s ) );
+											   ( kBytesWarmStart + kBytesSolve + kBytesRelax ) * nc + 3.0 * kBytesJoint * nj );
+		const FlowPlan plan = PlanFlow( StageChunks( xa.contactStart, xa.jointStart, xa.colors ), nj > 0 );
 		impl->Launch( kkSolveXcd, bytes, [&]( hipEvent_t e0, hipEvent_t e1 ) {
-			if ( e0 != nullptr )
-			{
-				HIP_CHECK( hipEventRecord( e0, s ) );
-			}
-			void* args[] = { &xa };
-			HIP_CHECK( hipLaunchCooperativeKernel( reinterpret_cast<const void*>( SolveXcdKernel ), dim3( kXcdGrid ), dim3( kXcdThreads ), args,
-												   0, s ) );
-			if ( e1 != nullptr )
-			{
-				HIP_CHECK( hipEventRecord( e1, s ) );
-			}
+			hipExtLaunchKernelGGL( plan.kernel, dim3( kFlowGrid ), dim3( plan.threads ), 0, s, e0, e1, 0, xa );
 		} );
+		if ( anyRestitution )
+		{
+			runStage( kStageRestitution );
+		}
 	}
-	else if ( fused )
+	else if ( solver == kSolverFused )
 	{
 		FusedArgs fa;
 		fa.color = ca;
@@ -5536,7 +6193,7 @@ void DeviceWorld::SolveFinish( FinalizeResult* result )
 		}
 		if ( mail[5] != 0 )
 		{
-			Fatal( "XCD solver: a barrier among its workgroups timed out (set B2AMD_NO_XCD_SOLVER to use the color kernels)" );
+			Fatal( "XCD solver: a wait among its workgroups timed out (set B2AMD_NO_XCD_SOLVER to use the other solvers)" );
 		}
 		result->enlargedBodies.assign( mail + kMailHeader, mail + kMailHeader + enlargedBodyCount );
 		result->enlargedShapes.assign( mail + pk.shapeOffset, mail + pk.shapeOffset + enlargedShapeCount );
@@ -5656,20 +6313,26 @@ void DeviceWorld::SetSolverPath( int path )
 	impl->solverPath = path;
 }
 
-bool DeviceWorld::WantsWarmLists( int bodyCount, int constraintCount, int activeColorCount, int overflowCount ) const
+bool DeviceWorld::WantsWarmLists( const SolverLists& lists ) const
 {
+	const int bodyCount = (int)lists.awakeBodies.size();
 	if ( bodyCount == 0 )
 	{
 		return false;
 	}
-	bool fits = bodyCount <= kFusedBodyCapacity && activeColorCount <= kMaxColorSlots;
-	bool fused = fits && ( impl->solverPath == 2 || ( impl->solverPath == 0 && AutoFused( constraintCount, overflowCount ) ) );
 	if ( impl->recording )
 	{
 		return BatchWarmByBody( bodyCount );
 	}
-	fused = fused || impl->tape != nullptr;
-	return WarmByBody( fused );
+	switch ( impl->tape != nullptr ? kSolverFused : ChooseSolver( impl->solverPath, lists, impl->XcdUsable() ) )
+	{
+		case kSolverFused:
+			return WarmByBody( true );
+		case kSolverXcd:
+			return false;
+		default:
+			return WarmByBody( false );
+	}
 }
 
 void DeviceWorld::SetTape( TapeStore* tape, int index )

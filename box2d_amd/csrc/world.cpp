@@ -4102,6 +4102,10 @@ static void BuildSolverLists( World& w, SolverLists& L )
 	// the awake order may have changed: the island slots go up again
 	w.islandsDirty = true;
 	L.awakeBodies = w.solverSets[kAwakeSet].bodyIds;
+	for ( int id : L.awakeBodies )
+	{
+		L.awakeKinematic = L.awakeKinematic || w.bodies[id].type == b2_kinematicBody;
+	}
 
 	for ( int i = 0; i < kGraphColorCount; ++i )
 	{
@@ -4352,10 +4356,8 @@ bool World::StepBegin( float timeStep, int subStepCount )
 		// A contact graph that stayed the same for two steps gets the per-body warm-start lists
 		// (worlds whose graph changes every step keep the color-by-color warm start).
 		listsStableSteps += 1;
-		int nb = (int)solverLists.awakeBodies.size();
 		if ( listsStableSteps >= 2 && solverLists.warmStart.empty() &&
-			 device->WantsWarmLists( nb, (int)solverLists.constraintContacts.size(), solverLists.activeColorCount,
-									 solverLists.overflowContactCount + solverLists.overflowJointCount ) )
+			 device->WantsWarmLists( solverLists ) )
 		{
 			BuildWarmLists( *this, solverLists );
 			device->UploadWarmLists( solverLists );

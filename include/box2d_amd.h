@@ -36,11 +36,12 @@ B2_API void b2amd_World_ResetKernelStats( b2WorldId worldId );
 /// Solver path of a world's step. The fused path runs the whole substep loop in one workgroup
 /// with the awake body states in LDS (up to 5400 awake bodies); the color-kernel path launches one
 /// kernel per graph color and stage; the XCD path runs the whole substep loop in one launch on the
-/// 32 compute units of one XCD, with a barrier among its workgroups between colors instead of
-/// kernel boundaries (MI355X only; worlds without overflow constraints). Auto picks the fused path
-/// for small worlds (up to 4096 contact constraints), else the color kernels. Results are
-/// bit-identical across paths; the switch exists for testing and measurement. Fused falls back to
-/// color kernels for worlds beyond its LDS budget, XCD to color kernels where it does not apply.
+/// 32 compute units of one XCD, each constraint waiting for its own two bodies (MI355X only; worlds
+/// without overflow constraints and awake kinematic bodies). Auto picks the fused path for small
+/// worlds, the XCD path for larger ones where it applies and, where it does not, the fused path up to
+/// 4096 contact constraints and the color kernels beyond. Results are bit-identical across paths;
+/// the switch exists for testing and measurement. Fused falls back to color kernels for worlds
+/// beyond its LDS budget, XCD to color kernels where it does not apply.
 typedef enum b2amd_SolverPath
 {
 	b2amd_solverAuto = 0,

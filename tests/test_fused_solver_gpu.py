@@ -1,7 +1,8 @@
-"""The single-workgroup solver's forms (rows resident in registers, rows streamed, general) against the
-color kernels, bit for bit after every step, at the sizes where a form's chunks change: one chunk per
-color, partial chunks, the last resident world and the first streamed one, several chunks of one color
-in a wavefront."""
+"""The single-workgroup solver's forms (rows resident in registers, rows streamed, general) and the XCD
+solver's (rows resident, more chunks than registers, joints) against the color kernels, bit for bit
+after every step, at the sizes where a form's chunks change: one chunk per color, partial chunks, the
+last resident world and the first streamed one, several chunks of one color in a wavefront, bodies
+without constraints."""
 
 import ctypes
 
@@ -78,4 +79,27 @@ def test_fused_matches_color_kernels(gpu_scenes, kind, size, materials, steps):
     colored, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
     assert kind == "chains" or contacts > 0
     for k, (a, b) in enumerate(zip(fused, colored)):
+        assert a == b, f"step {k + 2}"
+
+
+XCD_CASES = [("pyramid", rows, None, 20) for rows in (1, 2, 7, 25, 60)] + [("pyramid", 112, None, 6)]
+XCD_CASES += [("pile", n, m, 120) for n in (1, 65, 600) for m in ("rolling", "bouncy")]
+XCD_CASES += [("chains", 160, None, 40), ("rain", 17000, None, 3)]
+
+
+@pytest.mark.parametrize("kind,size,materials,steps", XCD_CASES)
+def test_xcd_matches_color_kernels(gpu_scenes, kind, size, materials, steps):
+    def make():
+        if kind == "pyramid":
+            return gpu_scenes.pyramid(size, 100.0)
+        if kind == "rain":
+            # spaced so that only a few neighbours touch: most bodies have no constraint
+            return gpu_scenes.create(box2d_amd.SCENE_RAIN, (size, 170, 0, 9), (136.0,))
+        if kind == "pile":
+            return gpu_scenes.create(box2d_amd.SCENE_MIXED_PILE, (size, 0, 78))
+        return gpu_scenes.create(box2d_amd.SCENE_BATCH_WORLD, (size, 2, 6))
+
+    xcd, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_XCD, steps, materials)
+    colored, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
+    for k, (a, b) in enumerate(zip(xcd, colored)):
         assert a == b, f"step {k + 2}"
