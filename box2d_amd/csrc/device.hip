@@ -1279,14 +1279,6 @@ struct FusedArgs
 	int warmByBody; // 1: warm start body by body, 0: color by color
 };
 
-// Workgroup barrier that orders LDS accesses only: global loads issued before it stay in flight.
-B2G_DEV void LdsBarrier()
-{
-	__builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup", "local" );
-	__builtin_amdgcn_s_barrier();
-	__builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "workgroup", "local" );
-}
-
 // LDS bytes of a world with `count` awake bodies: slot 0 holds the static identity state, slots
 // 1..count the awake bodies; 7 floats and 16 flag bits per slot.
 __host__ __device__ inline int FusedLdsBytes( int count )

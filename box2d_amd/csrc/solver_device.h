@@ -75,6 +75,14 @@ struct ConstraintSoA
 constexpr int kFusedBodyCapacity = 5400;
 constexpr int kStaticSlot = 0;
 
+// Workgroup barrier that orders LDS accesses only: global loads issued before it stay in flight.
+B2G_DEVI void LdsBarrier()
+{
+	__builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup", "local" );
+	__builtin_amdgcn_s_barrier();
+	__builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "workgroup", "local" );
+}
+
 B2G_DEVI float MaxW( float a, float b )
 {
 	return a >= b ? a : b;

@@ -1,0 +1,48 @@
+"""The backward kernel's two forms, a world's constraints one per thread (up to 256) and more than
+that, against the oracle's float64 reverse mode with the recorded branch pattern held fixed, to the
+1e-3 relative of the other adjoint checks."""
+
+import numpy as np
+import pytest
+
+from adjoint_ref import WorldRecord
+
+pytestmark = pytest.mark.gpu
+
+# rows, whether a step holds more than 256 constraints
+SIZES = [(2, False), (13, False), (14, True), (17, True)]
+
+
+@pytest.mark.parametrize("rows,large", SIZES)
+def test_backward_forms_match_fp64_adjoint(rows, large):
+    from box2d_amd.adjoint import BODY_STATE, PushWorlds
+
+    rng = np.random.default_rng(rows)
+    # fast pushers that hit within six steps, and a sixth of the horizon that the 1e-3 covers in the
+    # 10-row world, so that float32 rounding, which grows with the number of steps reversed, stays below
+    # it in the larger ones too (after 24 steps the 14-row world's is 1.3e-3)
+    params = np.stack([rng.uniform(5, 6, 2), rng.uniform(-0.5, 0.5, 2), rng.uniform(-1, 1, 2), rng.uniform(0.3, 0.9, 2)], 1)
+    goals = np.array([[0.5, rows - 1.0], [-0.5, rows - 0.5]])
+    steps = 10
+    pw = PushWorlds(params, rows=rows)
+    try:
+        tape = pw.record(steps)
+        most = max(int(tape.read_step(w, k)[0]["constraintCount"]) for w in range(2) for k in range(steps))
+        assert (most > 256) == large, most
+        final = tape.final_states()
+        # the loss looks at the box the pusher hits first: the first of the bottom row
+        target = [int(b[0]) for b in pw.body_ids]
+        fg = np.zeros((2, tape.body_stride), dtype=BODY_STATE)
+        for w in range(2):
+            fg[w]["center"][target[w]] = 2.0 * (final[w]["center"][target[w]] - goals[w])
+        ig, fr, stats = tape.backward(fg)
+        assert stats.unsupported == 0 and stats.replayMismatches == 0
+        shapes = pw.pusher_shape_ids()
+        for w in range(2):
+            pusher = int(pw.body_ids[w][-1])
+            got = np.array([*ig[w]["linearVelocity"][pusher], ig[w]["angularVelocity"][pusher], fr[w, shapes[w]]], dtype=np.float64)
+            rec = WorldRecord.from_tape(tape, w)
+            want, _ = rec.push_gradients(rec.slot_of(pusher), shapes[w], rec.slot_of(target[w]), goals[w])
+            assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want), (w, got, want)
+    finally:
+        pw.destroy()
