@@ -2230,8 +2230,8 @@ int b2amd_Tape_Backward( b2amd_Tape* tape, const b2amd_BodyState* finalGrad, b2a
 		args.push_back( a );
 	}
 
-	hipStream_t stream;
-	HIP_CHECK( hipStreamCreate( &stream ) );
+	int streamIndex = 0;
+	hipStream_t stream = AcquireWorldStream( &streamIndex );
 	hipEvent_t ev0, ev1;
 	HIP_CHECK( hipEventCreate( &ev0 ) );
 	HIP_CHECK( hipEventCreate( &ev1 ) );
@@ -2273,7 +2273,7 @@ int b2amd_Tape_Backward( b2amd_Tape* tape, const b2amd_BodyState* finalGrad, b2a
 	HIP_CHECK( hipEventElapsedTime( &ms, ev0, ev1 ) );
 	HIP_CHECK( hipEventDestroy( ev0 ) );
 	HIP_CHECK( hipEventDestroy( ev1 ) );
-	HIP_CHECK( hipStreamDestroy( stream ) );
+	ReleaseWorldStream( streamIndex );
 
 	hipFree( scratch );
 	hipFree( devSteps );

@@ -9,11 +9,18 @@
 #include <mutex>
 #include <vector>
 
+struct ihipStream_t;
+
 namespace b2g
 {
 
 class World;
 class TapeStore;
+
+// A stream shared by the worlds of the current device, and its return (device.hip).
+ihipStream_t* AcquireWorldStream( int* index );
+void ReleaseWorldStream( int index );
+
 
 // Work lists the host rebuilds when the set of awake bodies or the graph coloring changes.
 struct SolverLists
