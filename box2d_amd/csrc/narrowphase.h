@@ -823,8 +823,10 @@ B2G_DEV b2LocalManifold CollideSegmentAndPolygon( const b2Segment& segmentA, con
 }
 
 // Manifold dispatch for a primary-ordered shape pair (reference src/contact.c:188-206).
-// Chain segments are not handled here yet; the host refuses to create such contacts.
-B2G_DEV b2LocalManifold ComputeManifold( const ShapeDev& shapeA, const ShapeDev& shapeB, b2Transform xf )
+// Chain segments are not handled here yet; the host refuses to create such contacts. Shape is the world
+// step's record or the public one.
+template <typename Shape>
+B2G_DEV b2LocalManifold ComputeManifold( const Shape& shapeA, const Shape& shapeB, b2Transform xf )
 {
 	switch ( shapeA.type )
 	{

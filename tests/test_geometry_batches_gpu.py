@@ -1,0 +1,51 @@
+"""Batched manifolds, times of impact and distances at the counts where their split changes: part of a
+wavefront, whole ones, one chunk, two, all slots, slots used again. Every record gives what the
+reference's fixtures hold for it, bit for bit, whatever its place; a refused batch writes nothing."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import box2d_amd
+from b2types import DistanceInput, DistanceOutput, LocalManifold, Shape, SimplexCache, TOIInput, TOIOutput, Transform
+from b2types import manifold_array_words
+from test_manifolds import load_fixture
+from test_toi_fixture import check_toi, distance_words, load
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = [1, 63, 64, 65, 2879, 2881, 9000, 24001, 40000]
+
+
+def _take(ctype, records, index):
+    raw = np.frombuffer(bytes(records), dtype=np.uint8).reshape(-1, ctypes.sizeof(ctype))
+    return (ctype * len(index)).from_buffer_copy(raw[index].tobytes())
+
+
+@pytest.mark.parametrize("count", COUNTS)
+def test_manifolds(count):
+    a, b, x, want = load_fixture()
+    index = np.random.default_rng(count).integers(0, len(a), count)
+    lib = box2d_amd.library()
+    a, b, x, out = _take(Shape, a, index), _take(Shape, b, index), _take(Transform, x, index), (LocalManifold * count)()
+    assert lib.b2amd_CollideBatch(a, b, x, count, out) == 0
+    assert np.array_equal(manifold_array_words(out), want[index])
+    a[count - 1].type = 4  # chain segments are refused
+    before = ctypes.string_at(ctypes.byref(out), ctypes.sizeof(out))
+    assert lib.b2amd_CollideBatch(a, b, x, count, out) == -1
+    assert ctypes.string_at(ctypes.byref(out), ctypes.sizeof(out)) == before
+
+
+@pytest.mark.parametrize("count", COUNTS)
+def test_times_of_impact_and_distances(count):
+    n, toi_in, toi_out, dist_in, dist_out, dist_caches = load()
+    index = np.random.default_rng(count).integers(0, n, count)
+    lib = box2d_amd.library()
+    out = (TOIOutput * count)()
+    assert lib.b2amd_TimeOfImpactBatch(_take(TOIInput, toi_in, index), count, out) == 0
+    check_toi(bytes(out), toi_out[index])
+    out, caches = (DistanceOutput * count)(), (SimplexCache * count)()
+    assert lib.b2amd_ShapeDistanceBatch(_take(DistanceInput, dist_in, index), caches, count, out) == 0
+    assert np.array_equal(distance_words(bytes(out)), distance_words(dist_out[index].tobytes()))
+    assert bytes(caches) == dist_caches[index].tobytes()
