@@ -903,29 +903,34 @@ struct ColorRange
 };
 
 template <int Stage, typename Bodies>
+B2G_DEV void ColorJoint( const ColorArgs& a, JointSim* joint, const Bodies& B )
+{
+	if ( Stage == kStageWarmStart )
+	{
+		WarmStartJoint( joint, B );
+	}
+	else if ( Stage == kStageSolve )
+	{
+		// joint events: colored joints only, as the reference's overflow pass does not test
+		const bool events = ( joint->forceThreshold < FLT_MAX || joint->torqueThreshold < FLT_MAX ) && joint->eventFlag == 0;
+		SolveJoint( joint, B, true, a.p.h, a.p.inv_h );
+		if ( events && JointReactionReached( joint, a.p.inv_h ) )
+		{
+			joint->eventFlag = 1;
+		}
+	}
+	else if ( Stage == kStageRelax )
+	{
+		SolveJoint( joint, B, false, a.p.h, a.p.inv_h );
+	}
+}
+
+template <int Stage, typename Bodies>
 B2G_DEV void ColorLane( const ColorArgs& a, const ColorRange& r, int t, const Bodies& B )
 {
 	if ( t < r.jointCount )
 	{
-		JointSim* joint = a.joints + a.jointList[r.jointStart + t];
-		if ( Stage == kStageWarmStart )
-		{
-			WarmStartJoint( joint, B );
-		}
-		else if ( Stage == kStageSolve )
-		{
-			SolveJoint( joint, B, true, a.p.h, a.p.inv_h );
-			// joint events: colored joints only, as the reference's overflow pass does not test
-			if ( ( joint->forceThreshold < FLT_MAX || joint->torqueThreshold < FLT_MAX ) && joint->eventFlag == 0 &&
-				 JointReactionReached( joint, a.p.inv_h ) )
-			{
-				joint->eventFlag = 1;
-			}
-		}
-		else if ( Stage == kStageRelax )
-		{
-			SolveJoint( joint, B, false, a.p.h, a.p.inv_h );
-		}
+		ColorJoint<Stage>( a, a.joints + a.jointList[r.jointStart + t], B );
 		return;
 	}
 
@@ -1468,25 +1473,44 @@ B2G_DEV void FusedContactStage( const FusedArgs& a, const FusedLane& L, const Pa
 	// rows are loaded in one place, straight into the registers the next turn reads.
 	int color = 0;
 	int jointBase = L.waves >> 1;
+	int jointAhead = 0; // the lane's joint of the wavefront's first joint chunk in the color, loaded a color ahead
+	auto loadJointAhead = [&]() {
+		if ( kGeneral && L.anyJoints && color < L.colors )
+		{
+			int jointStart = __builtin_amdgcn_readlane( L.jointStarts, color );
+			int joints = __builtin_amdgcn_readlane( L.jointStarts, color + 1 ) - jointStart;
+			int t = 64 * ( ( L.wave - jointBase ) & ( L.waves - 1 ) ) + ( threadIdx.x & 63 );
+			if ( t < joints )
+			{
+				jointAhead = a.color.jointList[jointStart + t];
+			}
+		}
+	};
+	loadJointAhead();
 	auto passColor = [&]() {
 		int lanes = ColorContacts( L, color );
 		if ( kGeneral && L.anyJoints )
 		{
 			int jointStart = __builtin_amdgcn_readlane( L.jointStarts, color );
 			int joints = __builtin_amdgcn_readlane( L.jointStarts, color + 1 ) - jointStart;
-			for ( int k = ( L.wave - jointBase ) & ( L.waves - 1 ); 64 * k < joints; k += L.waves )
+			int t = 64 * ( ( L.wave - jointBase ) & ( L.waves - 1 ) ) + ( threadIdx.x & 63 );
+			if ( t < joints )
 			{
-				ColorRange range = { jointStart, joints, 0, 0 };
-				ColorLane<Stage>( a.color, range, 64 * k + ( threadIdx.x & 63 ), B );
+				ColorJoint<Stage>( a.color, a.color.joints + jointAhead, B );
+			}
+			for ( t += 64 * L.waves; t < joints; t += 64 * L.waves )
+			{
+				ColorJoint<Stage>( a.color, a.color.joints + a.color.jointList[jointStart + t], B );
 			}
 			jointBase += ( joints + 63 ) >> 6;
 			lanes += joints;
 		}
+		color = Uniform( color + 1 );
+		loadJointAhead();
 		if ( lanes > 0 )
 		{
 			LdsBarrier();
 		}
-		color = Uniform( color + 1 );
 	};
 	bool more = Uniform( q.color ) < L.colors;
 	while ( more )

@@ -22,6 +22,64 @@ namespace b2g
 // The device path runs with one length unit per meter (world creation rejects other settings).
 constexpr float kLengthUnitsPerMeter = 1.0f;
 
+// What a revolute joint's turn reads. Every turn loads it together with the joint's type, before the
+// branch on the type: a joint's record lies in L2, and with the loads behind the branch a turn waited
+// for two of its latencies (and for a third between the record's fields that stores to the record
+// might change). 24 x 24 bodies in a net of 1,104 joints: 133 us a step that way, 122 us this way.
+struct RevoluteRow
+{
+	int type;
+	int bodyA, bodyB; // in the solver's body view
+	float mA, mB, iA, iB;
+	Softness softness;
+	b2Vec2 impulse;
+	b2Transform frameA, frameB;
+	b2Vec2 deltaCenter;
+	int spring, motor, limit;
+
+	// All loads have arrived after this.
+	B2G_DEVI void Await()
+	{
+		asm volatile( "" : "+v"( type ), "+v"( bodyA ), "+v"( bodyB ), "+v"( mA ), "+v"( mB ), "+v"( iA ), "+v"( iB ),
+					  "+v"( softness.biasRate ), "+v"( softness.massScale ), "+v"( softness.impulseScale ) );
+		asm volatile( "" : "+v"( impulse.x ), "+v"( impulse.y ), "+v"( frameA.p.x ), "+v"( frameA.p.y ), "+v"( frameA.q.c ),
+					  "+v"( frameA.q.s ), "+v"( frameB.p.x ), "+v"( frameB.p.y ), "+v"( frameB.q.c ), "+v"( frameB.q.s ) );
+		asm volatile( "" : "+v"( deltaCenter.x ), "+v"( deltaCenter.y ), "+v"( spring ), "+v"( motor ), "+v"( limit ) );
+	}
+};
+
+template <typename Bodies>
+B2G_DEVI RevoluteRow LoadRevoluteRow( const JointSim* j )
+{
+	RevoluteRow r = { j->type,
+					  Bodies::JointA( j ),
+					  Bodies::JointB( j ),
+					  j->invMassA,
+					  j->invMassB,
+					  j->invIA,
+					  j->invIB,
+					  j->constraintSoftness,
+					  j->linearImpulse,
+					  j->frameA,
+					  j->frameB,
+					  j->deltaCenter,
+					  j->enableSpring,
+					  j->enableMotor,
+					  j->enableLimit };
+	r.Await();
+	return r;
+}
+
+B2G_DEVI void RevoluteWarmStartTerms( b2Vec2 impulse, float axialImpulse, b2Vec2 anchorA, b2Vec2 anchorB, b2Rot dqA, b2Rot dqB,
+									  b2Vec2& P, float& LA, float& LB )
+{
+	b2Vec2 rA = b2RotateVector( dqA, anchorA );
+	b2Vec2 rB = b2RotateVector( dqB, anchorB );
+	P = impulse;
+	LA = b2Cross( rA, impulse ) + axialImpulse;
+	LB = b2Cross( rB, impulse ) + axialImpulse;
+}
+
 // Warm-start impulses of one joint: body A receives v -= mA * P, w -= iA * LA and body B
 // v += mB * P, w += iB * LB. They depend on the accumulated impulses, the joint frames and the two
 // bodies' delta positions and rotations, never on velocities. Returns false for joints with no
@@ -33,12 +91,8 @@ B2G_DEVI bool JointWarmStartTerms( const JointSim* j, b2Rot dqA, b2Vec2 dpA, b2R
 	{
 		case b2_revoluteJoint:
 		{
-			b2Vec2 rA = b2RotateVector( dqA, j->frameA.p );
-			b2Vec2 rB = b2RotateVector( dqB, j->frameB.p );
 			float axialImpulse = j->springImpulse + j->motorImpulse + j->lowerImpulse - j->upperImpulse;
-			P = j->linearImpulse;
-			LA = b2Cross( rA, j->linearImpulse ) + axialImpulse;
-			LB = b2Cross( rB, j->linearImpulse ) + axialImpulse;
+			RevoluteWarmStartTerms( j->linearImpulse, axialImpulse, j->frameA.p, j->frameB.p, dqA, dqB, P, LA, LB );
 			return true;
 		}
 		case b2_weldJoint:
@@ -149,22 +203,34 @@ B2G_DEVI bool JointWarmStartTerms( const JointSim* j, b2Rot dqA, b2Vec2 dpA, b2R
 template <typename Bodies>
 B2G_DEVI void WarmStartJoint( JointSim* joint, const Bodies& B )
 {
-	int ia = Bodies::JointA( joint );
-	int ib = Bodies::JointB( joint );
+	float springImpulse = joint->springImpulse;
+	float motorImpulse = joint->motorImpulse;
+	float lowerImpulse = joint->lowerImpulse;
+	float upperImpulse = joint->upperImpulse;
+	const RevoluteRow r = LoadRevoluteRow<Bodies>( joint );
+	asm volatile( "" : "+v"( springImpulse ), "+v"( motorImpulse ), "+v"( lowerImpulse ), "+v"( upperImpulse ) );
+	int ia = r.bodyA;
+	int ib = r.bodyB;
 	BodyState sA = ToState( B.Load( ia ) );
 	BodyState sB = ToState( B.Load( ib ) );
 
 	b2Vec2 P;
 	float LA, LB;
-	if ( JointWarmStartTerms( joint, sA.deltaRotation, sA.deltaPosition, sB.deltaRotation, sB.deltaPosition, P, LA, LB ) == false )
+	if ( r.type == b2_revoluteJoint )
+	{
+		float axialImpulse = springImpulse + motorImpulse + lowerImpulse - upperImpulse;
+		RevoluteWarmStartTerms( r.impulse, axialImpulse, r.frameA.p, r.frameB.p, sA.deltaRotation, sB.deltaRotation, P, LA, LB );
+	}
+	else if ( JointWarmStartTerms( joint, sA.deltaRotation, sA.deltaPosition, sB.deltaRotation, sB.deltaPosition, P, LA, LB ) ==
+			  false )
 	{
 		return;
 	}
 
-	float mA = joint->invMassA;
-	float mB = joint->invMassB;
-	float iA = joint->invIA;
-	float iB = joint->invIB;
+	float mA = r.mA;
+	float mB = r.mB;
+	float iA = r.iA;
+	float iB = r.iB;
 	if ( sA.flags & kDynamicFlag )
 	{
 		sA.linearVelocity = b2MulSub( sA.linearVelocity, mA, P );
@@ -209,14 +275,14 @@ B2G_DEVI LimitRow MakeLimitRow( float C, float speculativeBias, bool useBias, co
 // Revolute
 
 template <typename Bodies>
-B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, float h, float inv_h )
+B2G_DEVI void SolveRevolute( JointSim* joint, const RevoluteRow& row, const Bodies& B, bool useBias, float h, float inv_h )
 {
-	float mA = joint->invMassA;
-	float mB = joint->invMassB;
-	float iA = joint->invIA;
-	float iB = joint->invIB;
-	int ia = Bodies::JointA( joint );
-	int ib = Bodies::JointB( joint );
+	float mA = row.mA;
+	float mB = row.mB;
+	float iA = row.iA;
+	float iB = row.iB;
+	int ia = row.bodyA;
+	int ib = row.bodyB;
 
 	BodyState sA = ToState( B.Load( ia ) );
 	BodyState* stateA = &sA;
@@ -228,13 +294,13 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 	b2Vec2 vB = stateB->linearVelocity;
 	float wB = stateB->angularVelocity;
 
-	b2Rot qA = b2MulRot( stateA->deltaRotation, joint->frameA.q );
-	b2Rot qB = b2MulRot( stateB->deltaRotation, joint->frameB.q );
+	b2Rot qA = b2MulRot( stateA->deltaRotation, row.frameA.q );
+	b2Rot qB = b2MulRot( stateB->deltaRotation, row.frameB.q );
 	b2Rot relQ = b2InvMulRot( qA, qB );
 
 	bool fixedRotation = ( iA + iB == 0.0f );
 
-	if ( joint->enableSpring && fixedRotation == false )
+	if ( row.spring && fixedRotation == false )
 	{
 		float jointAngle = Atan2( relQ.s, relQ.c );
 		float jointAngleDelta = b2UnwindAngle( jointAngle - joint->targetAngle );
@@ -249,7 +315,7 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 		wB += iB * impulse;
 	}
 
-	if ( joint->enableMotor && fixedRotation == false )
+	if ( row.motor && fixedRotation == false )
 	{
 		float Cdot = wB - wA - joint->motorSpeed;
 		float impulse = -joint->axialMass * Cdot;
@@ -261,13 +327,13 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 		wB += iB * impulse;
 	}
 
-	if ( joint->enableLimit && fixedRotation == false )
+	if ( row.limit && fixedRotation == false )
 	{
 		float jointAngle = Atan2( relQ.s, relQ.c );
 
 		{
 			float C = jointAngle - joint->lowerAngle;
-			LimitRow r = MakeLimitRow( C, C * inv_h, useBias, joint->constraintSoftness );
+			LimitRow r = MakeLimitRow( C, C * inv_h, useBias, row.softness );
 			float Cdot = wB - wA;
 			float oldImpulse = joint->lowerImpulse;
 			float impulse = -r.massScale * joint->axialMass * ( Cdot + r.bias ) - r.impulseScale * oldImpulse;
@@ -279,7 +345,7 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 
 		{
 			float C = joint->upperAngle - jointAngle;
-			LimitRow r = MakeLimitRow( C, C * inv_h, useBias, joint->constraintSoftness );
+			LimitRow r = MakeLimitRow( C, C * inv_h, useBias, row.softness );
 			float Cdot = wA - wB;
 			float oldImpulse = joint->upperImpulse;
 			float impulse = -r.massScale * joint->axialMass * ( Cdot + r.bias ) - r.impulseScale * oldImpulse;
@@ -291,8 +357,8 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 	}
 
 	{
-		b2Vec2 rA = b2RotateVector( stateA->deltaRotation, joint->frameA.p );
-		b2Vec2 rB = b2RotateVector( stateB->deltaRotation, joint->frameB.p );
+		b2Vec2 rA = b2RotateVector( stateA->deltaRotation, row.frameA.p );
+		b2Vec2 rB = b2RotateVector( stateB->deltaRotation, row.frameB.p );
 
 		b2Vec2 Cdot = b2Sub( b2Add( vB, b2CrossSV( wB, rB ) ), b2Add( vA, b2CrossSV( wA, rA ) ) );
 
@@ -303,10 +369,10 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 		{
 			b2Vec2 dcA = stateA->deltaPosition;
 			b2Vec2 dcB = stateB->deltaPosition;
-			b2Vec2 separation = b2Add( b2Add( b2Sub( dcB, dcA ), b2Sub( rB, rA ) ), joint->deltaCenter );
-			bias = b2MulSV( joint->constraintSoftness.biasRate, separation );
-			massScale = joint->constraintSoftness.massScale;
-			impulseScale = joint->constraintSoftness.impulseScale;
+			b2Vec2 separation = b2Add( b2Add( b2Sub( dcB, dcA ), b2Sub( rB, rA ) ), row.deltaCenter );
+			bias = b2MulSV( row.softness.biasRate, separation );
+			massScale = row.softness.massScale;
+			impulseScale = row.softness.impulseScale;
 		}
 
 		b2Mat22 K;
@@ -317,10 +383,10 @@ B2G_DEVI void SolveRevolute( JointSim* joint, const Bodies& B, bool useBias, flo
 		b2Vec2 b = b2Solve22( K, b2Add( Cdot, bias ) );
 
 		b2Vec2 impulse;
-		impulse.x = -massScale * b.x - impulseScale * joint->linearImpulse.x;
-		impulse.y = -massScale * b.y - impulseScale * joint->linearImpulse.y;
-		joint->linearImpulse.x += impulse.x;
-		joint->linearImpulse.y += impulse.y;
+		impulse.x = -massScale * b.x - impulseScale * row.impulse.x;
+		impulse.y = -massScale * b.y - impulseScale * row.impulse.y;
+		joint->linearImpulse.x = row.impulse.x + impulse.x;
+		joint->linearImpulse.y = row.impulse.y + impulse.y;
 
 		vA = b2MulSub( vA, mA, impulse );
 		wA -= iA * b2Cross( rA, impulse );
@@ -1308,10 +1374,11 @@ B2G_DEVI bool JointReactionReached( const JointSim* j, float inv_h )
 template <typename Bodies>
 B2G_DEVI void SolveJoint( JointSim* joint, const Bodies& B, bool useBias, float h, float inv_h )
 {
-	switch ( joint->type )
+	const RevoluteRow row = LoadRevoluteRow<Bodies>( joint );
+	switch ( row.type )
 	{
 		case b2_revoluteJoint:
-			SolveRevolute( joint, B, useBias, h, inv_h );
+			SolveRevolute( joint, row, B, useBias, h, inv_h );
 			break;
 		case b2_weldJoint:
 			SolveWeld( joint, B, useBias );

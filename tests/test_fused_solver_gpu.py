@@ -63,7 +63,7 @@ def _run(scenes, make, path, steps, materials):
 
 CASES = [("pyramid", rows, None, 40) for rows in (1, 2, 7, 11, 16, 21, 22, 23, 24, 25, 40)]
 CASES += [("pile", n, m, 150) for n in (1, 3, 33, 130) for m in (None, "rolling", "bouncy")]
-CASES += [("pile", 600, "rolling", 200), ("chains", 160, None, 40)]
+CASES += [("pile", 600, "rolling", 200), ("chains", 8, None, 40), ("chains", 160, None, 40), ("chains", 2600, None, 10)]
 
 
 @pytest.mark.parametrize("kind,size,materials,steps", CASES)
