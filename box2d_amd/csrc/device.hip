@@ -1251,7 +1251,7 @@ __global__ __launch_bounds__( kOverflowThreads ) void OverflowLevelKernel( Color
 // against one lane per constraint with every field loaded in its phase: 20-row pyramid (590 contacts,
 // 9 colors, resident) 202 -> 48 us; 1000-body mixed pile (about 3000 contacts, 13 colors, streamed)
 // 290 -> 190 us, then bound by its CU's vector instructions; 24x24 net of revolute joints (general)
-// 154 -> 135 us, bound by the joints' scattered loads.
+// 154 -> 122 us, bound by the latency of the joints' scattered loads.
 
 constexpr int kFusedThreads = 1024;
 constexpr int kFusedMaxContacts = 4096;
@@ -5742,7 +5742,7 @@ enum SolverKind
 // path: b2amd_SolverPath. Auto takes the fused solver while a stage's chunks fit its wavefronts (the
 // resident form: measured 48 us per step for the 20-row pyramid, 55 for 24 rows, 64 for a 400-body
 // pile, against 65, 66 and 82 in the XCD solver), above that the XCD solver where it applies (26 rows
-// 66 against 120 us, 500 bodies 85 against 167, a 40x40 joint net 151 against 254; 100 rows 88 against
+// 66 against 120 us, 500 bodies 85 against 167, a 40x40 joint net 148 against 225; 100 rows 88 against
 // 279 in the color kernels, 20,000 bodies 288 against 689). Worlds it does not apply to (overflow
 // constraints, awake kinematic bodies) keep the fused solver up to kFusedMaxContacts contacts, where
 // its one launch beats the color kernels' about 70, and the color kernels beyond.
