@@ -2230,6 +2230,7 @@ int b2amd_Tape_Backward( b2amd_Tape* tape, const b2amd_BodyState* finalGrad, b2a
 		args.push_back( a );
 	}
 
+	AwaitDefaultStream();
 	int streamIndex = 0;
 	hipStream_t stream = AcquireWorldStream( &streamIndex );
 	hipEvent_t ev0, ev1;

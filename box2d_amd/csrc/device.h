@@ -20,7 +20,7 @@ class TapeStore;
 // A stream shared by the worlds of the current device, and its return (device.hip).
 ihipStream_t* AcquireWorldStream( int* index );
 void ReleaseWorldStream( int index );
-
+void AwaitDefaultStream();
 
 // Work lists the host rebuilds when the set of awake bodies or the graph coloring changes.
 struct SolverLists

@@ -4571,6 +4571,14 @@ hipStream_t AcquireWorldStream( int* index )
 	return w.stream[k];
 }
 
+// A caller's host arrays may be pinned, and earlier work on the default stream or on a stream that waits
+// for it may still be about to write them. The worlds' streams do not wait for either, so calls that
+// take host arrays wait here before they read them.
+void AwaitDefaultStream()
+{
+	HIP_CHECK( hipStreamSynchronize( nullptr ) );
+}
+
 void ReleaseWorldStream( int index )
 {
 	std::lock_guard<std::mutex> lock( s_streamMutex );
@@ -6847,8 +6855,8 @@ struct GeometryArray
 	size_t size; // of a record
 };
 
-// Run launch( arrays in the slot, records, stream ) over the records, a slot's worth at a time. Calls
-// take turns.
+// Run launch( arrays in the slot, records, stream ) over the records, a slot's worth at a time, after
+// the work that the default stream waits for (see AwaitDefaultStream). Calls take turns.
 template <int kArrays, typename Launch>
 static void RunGeometry( const GeometryArray ( &arrays )[kArrays], int count, Launch launch )
 {
@@ -6861,6 +6869,7 @@ static void RunGeometry( const GeometryArray ( &arrays )[kArrays], int count, La
 	const int quarter = std::max( ( count - 1 ) / kGeometrySlots + 1, (int)( kGeometryLeastBytes / pairBytes ) );
 	const int most = std::min( ( quarter + kGeometryLanes - 1 ) / kGeometryLanes, (int)( kGeometrySlotBytes / pairBytes ) / kGeometryLanes ) *
 					 kGeometryLanes;
+	AwaitDefaultStream();
 	std::lock_guard<std::mutex> lock( s_geometry.mutex );
 	if ( s_geometry.ptr == nullptr )
 	{

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from adjoint_ref import WorldRecord
+from earlier_work import EarlierWork
 
 pytestmark = pytest.mark.gpu
 
@@ -44,5 +45,27 @@ def test_backward_forms_match_fp64_adjoint(rows, large):
             rec = WorldRecord.from_tape(tape, w)
             want, _ = rec.push_gradients(rec.slot_of(pusher), shapes[w], rec.slot_of(target[w]), goals[w])
             assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want), (w, got, want)
+    finally:
+        pw.destroy()
+
+
+@pytest.mark.parametrize("blocking", [False, True])
+def test_final_gradient_written_by_earlier_work(blocking):
+    import ctypes
+
+    from box2d_amd.adjoint import BODY_STATE, PushWorlds
+
+    pw = PushWorlds(np.array([[5.0, 0.1, 0.3, 0.5]]), rows=3)
+    try:
+        tape = pw.record(8)
+        fg = np.zeros((1, tape.body_stride), dtype=BODY_STATE)
+        fg["center"] = np.random.default_rng(1).uniform(-1, 1, (1, tape.body_stride, 2))
+        want, _, _ = tape.backward(fg)
+        assert np.any(want["linearVelocity"] != 0)
+        with EarlierWork(blocking) as work:
+            got = np.zeros_like(want)
+            records = (ctypes.c_byte * fg.nbytes).from_buffer_copy(fg.tobytes())
+            assert tape.lib.b2amd_Tape_Backward(tape.handle, work.writes(records), got.ctypes.data_as(ctypes.c_void_p), None, None) == 0
+        assert got.tobytes() == want.tobytes()
     finally:
         pw.destroy()

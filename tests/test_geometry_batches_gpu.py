@@ -1,6 +1,7 @@
 """Batched manifolds, times of impact and distances at the counts where their split changes: part of a
 wavefront, whole ones, one chunk, two, all slots, slots used again. Every record gives what the
-reference's fixtures hold for it, bit for bit, whatever its place; a refused batch writes nothing."""
+reference's fixtures hold for it, bit for bit, whatever its place; a refused batch writes nothing; inputs
+that earlier work on the device is still about to write are read after it."""
 
 import ctypes
 
@@ -10,6 +11,7 @@ import pytest
 import box2d_amd
 from b2types import DistanceInput, DistanceOutput, LocalManifold, Shape, SimplexCache, TOIInput, TOIOutput, Transform
 from b2types import manifold_array_words
+from earlier_work import EarlierWork
 from test_manifolds import load_fixture
 from test_toi_fixture import check_toi, distance_words, load
 
@@ -49,3 +51,22 @@ def test_times_of_impact_and_distances(count):
     assert lib.b2amd_ShapeDistanceBatch(_take(DistanceInput, dist_in, index), caches, count, out) == 0
     assert np.array_equal(distance_words(bytes(out)), distance_words(dist_out[index].tobytes()))
     assert bytes(caches) == dist_caches[index].tobytes()
+
+
+@pytest.mark.parametrize("blocking", [False, True])
+def test_inputs_written_by_earlier_work(blocking):
+    n, toi_in, toi_out, dist_in, dist_out, _ = load()
+    a, b, x, want = load_fixture()
+    lib = box2d_amd.library()
+    with EarlierWork(blocking) as work:
+        out = (TOIOutput * n)()
+        assert lib.b2amd_TimeOfImpactBatch(work.writes(toi_in), n, out) == 0
+        check_toi(bytes(out), toi_out)
+        out, caches = (DistanceOutput * n)(), (SimplexCache * n)()
+        assert lib.b2amd_ShapeDistanceBatch(work.writes(dist_in), caches, n, out) == 0
+        assert np.array_equal(distance_words(bytes(out)), distance_words(dist_out.tobytes()))
+        index = np.arange(9000) % len(a)
+        a, b, x = _take(Shape, a, index), _take(Shape, b, index), _take(Transform, x, index)
+        out = (LocalManifold * len(index))()
+        assert lib.b2amd_CollideBatch(a, b, work.writes(x), len(index), out) == 0
+        assert np.array_equal(manifold_array_words(out), want[index])
