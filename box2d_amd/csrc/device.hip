@@ -4592,8 +4592,10 @@ DeviceWorld::DeviceWorld()
 	impl = new Impl();
 	impl->stream = AcquireWorldStream( &impl->streamIndex );
 	impl->counters = static_cast<int*>( s_devicePool.Alloc( 16 * sizeof( int ) ) );
-	// zero once: from then on the pack kernels clear the counters after reading them
-	HIP_CHECK( hipMemset( impl->counters, 0, 16 * sizeof( int ) ) );
+	// zero once: from then on the pack kernels clear the counters after reading them. Waited for: a
+	// batch's kernels, on a stream of their own, may be the first to count.
+	HIP_CHECK( hipMemsetAsync( impl->counters, 0, 16 * sizeof( int ), impl->stream ) );
+	HIP_CHECK( hipStreamSynchronize( impl->stream ) );
 	impl->hostCounters = static_cast<int*>( s_pinnedPool.Alloc( 16 * sizeof( int ) ) );
 	for ( int i = 0; i < 4; ++i )
 	{
@@ -4930,6 +4932,10 @@ void DeviceWorld::UploadContinuousFilterRejects( const std::vector<uint64_t>& ke
 		return;
 	}
 	UploadVector( impl->ccdFilterRejects, keys, impl->stream );
+	if ( impl->recording )
+	{
+		HIP_CHECK( hipStreamSynchronize( impl->stream ) ); // a batch's kernels run on another stream
+	}
 	impl->ccdFilterRejectCount = (int)keys.size();
 }
 
@@ -6489,8 +6495,10 @@ void DeviceWorld::UploadIslands( const std::vector<int>& slots, const std::vecto
 	impl->islandBits.Reserve( std::max<size_t>( words, 1 ), false, impl->stream, 0 );
 	if ( impl->islandBits.capacity > impl->islandBitsZeroed )
 	{
-		// the pack kernel clears the words it reads; fresh storage starts at zero once
+		// the pack kernel clears the words it reads; fresh storage starts at zero once (waited for: a
+		// batch's kernels run on another stream)
 		HIP_CHECK( hipMemsetAsync( impl->islandBits.ptr, 0, impl->islandBits.capacity * sizeof( uint32_t ), impl->stream ) );
+		HIP_CHECK( hipStreamSynchronize( impl->stream ) );
 		impl->islandBitsZeroed = impl->islandBits.capacity;
 	}
 	impl->islandCount = islandCount;

@@ -1,13 +1,15 @@
 """Worlds share streams and memory blocks: more worlds than streams, made, stepped and dropped from
-several threads, each end bit for bit as a world that runs alone; and transforms of more bodies than one
-readback holds."""
+several threads, or while the default stream is busy, each end bit for bit as a world that runs alone; and
+transforms of more bodies than one readback holds."""
 
+import ctypes
 import threading
 
 import numpy as np
 import pytest
 
 import box2d_amd
+from earlier_work import EarlierWork
 
 pytestmark = pytest.mark.gpu
 
@@ -62,6 +64,29 @@ def test_worlds_made_and_dropped_in_threads(gpu_scenes, threads, worlds, sizes):
     for t in pool:
         t.join()
     assert wrong == []
+
+
+@pytest.mark.parametrize("together", [False, True])
+def test_worlds_made_while_the_default_stream_is_busy(gpu_scenes, together):
+    steps, sizes = 30, (1, 40, 130, 300)
+
+    def run():
+        worlds = [gpu_scenes.create(box2d_amd.SCENE_MIXED_PILE, (n, 1, 77)) for n in sizes]
+        ids = (box2d_amd.WorldId * len(worlds))(*[gpu_scenes.world_id(h) for h in worlds])
+        if together:
+            box2d_amd.step_worlds(ids, steps)
+        else:
+            for h in worlds:
+                gpu_scenes.step(h, steps)
+        out = [(_state(gpu_scenes, h), gpu_scenes.counters(h)) for h in worlds]
+        for h in worlds:
+            gpu_scenes.destroy(h)
+        return out
+
+    want = run()
+    with EarlierWork(False) as work:
+        work.writes((ctypes.c_int * 16)())
+        assert run() == want
 
 
 @pytest.mark.parametrize("rows", [457, 458])  # 104,653 and 105,111 boxes; one readback holds 104,857
