@@ -4481,6 +4481,11 @@ struct DeviceWorld::Impl
 		}
 		size_t cap = std::max<size_t>( n, constraintCapacity + constraintCapacity / 2 );
 		cap = std::max<size_t>( cap, 64 );
+		if ( cfields.ptr != nullptr )
+		{
+			// another world may take the blocks at once
+			HIP_CHECK( hipDeviceSynchronize() );
+		}
 		cfields.Free();
 		cints.Free();
 		cfields.Reserve( cap * kcFieldCount, false, stream, 0 );
