@@ -6729,15 +6729,27 @@ int DeviceWorld::AwakeBodyCount() const
 // launches a kernel that reads them there over the bus, a wavefront fetching its 64 records as whole
 // 16-byte words, all in flight together, into LDS (the lanes' own reads of a record would each cross
 // the bus alone), and writes its results back the same way; meanwhile the host fills the next slot.
-// Slots of 0.5, 1 and 2 MB: 32,768 manifolds in 858, 752 and 668 us (copies to and from device buffers
-// by the runtime: 768). Fewer than 1 MB of records stay one chunk: 4,096 distances (0.9 MB) take 67 us
-// in one and 77 in four. Converting the shapes on the host and copying through device buffers took
-// 1,640 to 3,600 us and 108 us.
+// Slots of 0.5, 1 and 2 MB: 32,768 manifolds in 858, 752 and 668 us. Fewer than 1 MB of records stay one
+// chunk: 4,096 distances (0.9 MB) take 67 us in one and 77 in four. Converting the shapes on the host and
+// copying through device buffers took 1,640 to 3,600 us and 108 us.
+//
+// The host's core copies every byte in and out, which the runtime's copies of whole arrays to and from
+// device memory do faster; what they cost on top (an allocation, a wait per array) is some 70 us plus the
+// time that the slots overlap. So calls above a size go that way. Measured with arrays read just before /
+// new ones, us, slots against device memory: times of impact, which keep the slots' kernels busy longest,
+// 40,000 in 458/538 against 464/557, 50,000 573/681 and 575/685, 60,000 685/839 and 652/784, 262,144
+// 3,888/3,916 and 2,937/2,954; distances 90,000 in 777/971 against 839/994, 110,000 958/1,222 and
+// 975/1,133, 262,144 3,008/3,149 and 2,608/2,593; manifolds 60,000 in 1,198/1,890 against 1,169/2,074,
+// 90,000 2,566/2,846 and 2,124/3,055, 262,144 8,753/8,841 and 8,310/8,604.
 
 constexpr int kGeometryLanes = 64;		  // a workgroup: one wavefront, a record per lane
 constexpr int kGeometrySlots = 4;		  // chunks in flight
 constexpr size_t kGeometrySlotBytes = 2 << 20;
 constexpr size_t kGeometryLeastBytes = 1 << 20; // of a chunk, when there are several
+// records of a call that still go through the slots
+constexpr size_t kTimeOfImpactPinnedBytes = 12 << 20; // 49,932
+constexpr size_t kDistancePinnedBytes = 20 << 20;	  // 100,824
+constexpr size_t kManifoldPinnedBytes = 32 << 20;	  // 92,182
 
 // The wavefront's 64 records (fewer at the end) on their way to LDS.
 template <typename T>
@@ -6868,15 +6880,53 @@ struct GeometryArray
 	size_t size; // of a record
 };
 
-// Run launch( arrays in the slot, records, stream ) over the records, a slot's worth at a time, after
-// the work that the default stream waits for (see AwaitDefaultStream). Calls take turns.
+// The whole arrays through device memory, by the runtime's copies (on the default stream).
 template <int kArrays, typename Launch>
-static void RunGeometry( const GeometryArray ( &arrays )[kArrays], int count, Launch launch )
+static void RunGeometryInDeviceMemory( const GeometryArray ( &arrays )[kArrays], int count, Launch launch )
+{
+	size_t offset[kArrays + 1] = {};
+	for ( int k = 0; k < kArrays; ++k )
+	{
+		offset[k + 1] = offset[k] + ( ( count * arrays[k].size + 255 ) & ~(size_t)255 );
+	}
+	char* base = nullptr;
+	HIP_CHECK( hipMalloc( &base, offset[kArrays] ) );
+	char* at[kArrays];
+	for ( int k = 0; k < kArrays; ++k )
+	{
+		at[k] = base + offset[k];
+		if ( arrays[k].in != nullptr )
+		{
+			HIP_CHECK( hipMemcpy( at[k], arrays[k].in, count * arrays[k].size, hipMemcpyHostToDevice ) );
+		}
+	}
+	launch( at, count, nullptr );
+	HIP_CHECK( hipGetLastError() );
+	for ( int k = 0; k < kArrays; ++k )
+	{
+		if ( arrays[k].out != nullptr )
+		{
+			HIP_CHECK( hipMemcpy( arrays[k].out, at[k], count * arrays[k].size, hipMemcpyDeviceToHost ) );
+		}
+	}
+	HIP_CHECK( hipFree( base ) );
+}
+
+// Run launch( arrays in the slot, records, stream ) over the records, a slot's worth at a time, after
+// the work that the default stream waits for (see AwaitDefaultStream); more than pinnedBytes of records
+// through device memory instead. Calls take turns.
+template <int kArrays, typename Launch>
+static void RunGeometry( const GeometryArray ( &arrays )[kArrays], int count, size_t pinnedBytes, Launch launch )
 {
 	size_t pairBytes = 0;
 	for ( const GeometryArray& a : arrays )
 	{
 		pairBytes += a.size;
+	}
+	if ( count * pairBytes > pinnedBytes )
+	{
+		RunGeometryInDeviceMemory( arrays, count, launch );
+		return;
 	}
 	// a chunk for each slot, of kGeometryLeastBytes to kGeometrySlotBytes, whole wavefronts
 	const int quarter = std::max( ( count - 1 ) / kGeometrySlots + 1, (int)( kGeometryLeastBytes / pairBytes ) );
@@ -6957,7 +7007,7 @@ int TimeOfImpactBatch( const b2TOIInput* inputs, int count, b2TOIOutput* outputs
 		return 0;
 	}
 	const GeometryArray arrays[2] = { { inputs, nullptr, sizeof( b2TOIInput ) }, { nullptr, outputs, sizeof( b2TOIOutput ) } };
-	RunGeometry( arrays, count, []( char** at, int n, hipStream_t stream ) {
+	RunGeometry( arrays, count, kTimeOfImpactPinnedBytes, []( char** at, int n, hipStream_t stream ) {
 		TimeOfImpactBatchKernel<<<GeometryBlocks( n ), kGeometryLanes, 0, stream>>>(
 			reinterpret_cast<const b2TOIInput*>( at[0] ), n, reinterpret_cast<b2TOIOutput*>( at[1] ) );
 	} );
@@ -6973,7 +7023,7 @@ int ShapeDistanceBatch( const b2DistanceInput* inputs, b2SimplexCache* caches, i
 	const GeometryArray arrays[3] = { { inputs, nullptr, sizeof( b2DistanceInput ) },
 									  { caches, caches, sizeof( b2SimplexCache ) },
 									  { nullptr, outputs, sizeof( b2DistanceOutput ) } };
-	RunGeometry( arrays, count, []( char** at, int n, hipStream_t stream ) {
+	RunGeometry( arrays, count, kDistancePinnedBytes, []( char** at, int n, hipStream_t stream ) {
 		ShapeDistanceBatchKernel<<<GeometryBlocks( n ), kGeometryLanes, 0, stream>>>(
 			reinterpret_cast<const b2DistanceInput*>( at[0] ), reinterpret_cast<b2SimplexCache*>( at[1] ), n,
 			reinterpret_cast<b2DistanceOutput*>( at[2] ) );
@@ -7110,7 +7160,7 @@ int CollideBatch( const b2amd_Shape* shapesA, const b2amd_Shape* shapesB, const 
 									  { shapesB, nullptr, sizeof( b2amd_Shape ) },
 									  { transforms, nullptr, sizeof( b2Transform ) },
 									  { nullptr, manifolds, sizeof( b2LocalManifold ) } };
-	RunGeometry( arrays, count, []( char** at, int n, hipStream_t stream ) {
+	RunGeometry( arrays, count, kManifoldPinnedBytes, []( char** at, int n, hipStream_t stream ) {
 		CollideBatchKernel<<<GeometryBlocks( n ), kGeometryLanes, 0, stream>>>(
 			reinterpret_cast<const b2amd_Shape*>( at[0] ), reinterpret_cast<const b2amd_Shape*>( at[1] ),
 			reinterpret_cast<const b2Transform*>( at[2] ), n, reinterpret_cast<b2LocalManifold*>( at[3] ) );

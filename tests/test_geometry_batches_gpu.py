@@ -1,7 +1,7 @@
 """Batched manifolds, times of impact and distances at the counts where their split changes: part of a
-wavefront, whole ones, one chunk, two, all slots, slots used again. Every record gives what the
-reference's fixtures hold for it, bit for bit, whatever its place; a refused batch writes nothing; inputs
-that earlier work on the device is still about to write are read after it."""
+wavefront, whole ones, one chunk, two, all slots, slots used again, whole arrays in device memory. Every
+record gives what the reference's fixtures hold for it, bit for bit, whatever its place; a refused batch
+writes nothing; inputs that earlier work on the device is still about to write are read after it."""
 
 import ctypes
 
@@ -17,7 +17,11 @@ from test_toi_fixture import check_toi, distance_words, load
 
 pytestmark = pytest.mark.gpu
 
+# the last ones on either side of where the arrays go through device memory
 COUNTS = [1, 63, 64, 65, 2879, 2881, 9000, 24001, 40000]
+MANIFOLD_COUNTS = COUNTS + [92182, 92183]
+TOI_COUNTS = COUNTS + [49932, 49933]
+DISTANCE_COUNTS = COUNTS + [100824, 100825, 150001]
 
 
 def _take(ctype, records, index):
@@ -25,7 +29,7 @@ def _take(ctype, records, index):
     return (ctype * len(index)).from_buffer_copy(raw[index].tobytes())
 
 
-@pytest.mark.parametrize("count", COUNTS)
+@pytest.mark.parametrize("count", MANIFOLD_COUNTS)
 def test_manifolds(count):
     a, b, x, want = load_fixture()
     index = np.random.default_rng(count).integers(0, len(a), count)
@@ -39,15 +43,21 @@ def test_manifolds(count):
     assert ctypes.string_at(ctypes.byref(out), ctypes.sizeof(out)) == before
 
 
-@pytest.mark.parametrize("count", COUNTS)
-def test_times_of_impact_and_distances(count):
-    n, toi_in, toi_out, dist_in, dist_out, dist_caches = load()
+@pytest.mark.parametrize("count", TOI_COUNTS)
+def test_times_of_impact(count):
+    n, toi_in, toi_out, _, _, _ = load()
     index = np.random.default_rng(count).integers(0, n, count)
-    lib = box2d_amd.library()
     out = (TOIOutput * count)()
-    assert lib.b2amd_TimeOfImpactBatch(_take(TOIInput, toi_in, index), count, out) == 0
+    assert box2d_amd.library().b2amd_TimeOfImpactBatch(_take(TOIInput, toi_in, index), count, out) == 0
     check_toi(bytes(out), toi_out[index])
+
+
+@pytest.mark.parametrize("count", DISTANCE_COUNTS)
+def test_distances(count):
+    n, _, _, dist_in, dist_out, dist_caches = load()
+    index = np.random.default_rng(count).integers(0, n, count)
     out, caches = (DistanceOutput * count)(), (SimplexCache * count)()
+    lib = box2d_amd.library()
     assert lib.b2amd_ShapeDistanceBatch(_take(DistanceInput, dist_in, index), caches, count, out) == 0
     assert np.array_equal(distance_words(bytes(out)), distance_words(dist_out[index].tobytes()))
     assert bytes(caches) == dist_caches[index].tobytes()
