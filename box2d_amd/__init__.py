@@ -93,6 +93,18 @@ def set_solver_path(world_id, path):
     library().b2amd_World_SetSolverPath(world_id, ctypes.c_int(path))
 
 
+class SolverInfo(ctypes.Structure):
+    """b2amd_SolverInfo (include/box2d_amd.h): how a world's last substep loop ran."""
+    _fields_ = [("path", ctypes.c_int), ("form", ctypes.c_int), ("threads", ctypes.c_int), ("chunks", ctypes.c_int)]
+
+
+def last_solver(world_id):
+    """The SolverInfo of a world's last step."""
+    f = library().b2amd_World_GetLastSolver
+    f.restype, f.argtypes = SolverInfo, [WorldId]
+    return f(world_id)
+
+
 def scenes():
     """Scene driver bound to the GPU library."""
     library()

@@ -1983,6 +1983,12 @@ int b2amd_World_GetLastPairQuery( b2WorldId worldId )
 	return world != nullptr ? world->lastPairQueryPath : 0;
 }
 
+b2amd_SolverInfo b2amd_World_GetLastSolver( b2WorldId worldId )
+{
+	World* world = GetWorld( worldId );
+	return world != nullptr ? world->device->LastSolver() : b2amd_SolverInfo{};
+}
+
 int b2amd_TimeOfImpactBatch( const b2TOIInput* inputs, int count, b2TOIOutput* outputs )
 {
 	return TimeOfImpactBatch( inputs, count, outputs );

@@ -3,6 +3,7 @@
 // compiles without HIP headers.
 #pragma once
 
+#include "box2d_amd.h"
 #include "layout.h"
 
 #include <cstdint>
@@ -216,6 +217,7 @@ public:
 
 	// Solver path: 0 auto, 1 color kernels, 2 fused when the world fits.
 	void SetSolverPath( int path );
+	b2amd_SolverInfo LastSolver() const;
 	// Whether the next solve of a world with these list sizes takes the color-kernel path with the
 	// warm start body by body (the host then builds the per-body warm-start lists).
 	bool WantsWarmLists( const SolverLists& lists ) const;

@@ -1874,15 +1874,17 @@ static int StageChunks( const Starts& contactStart, const Starts& jointStart, in
 
 constexpr int kFusedResidentChunks = kResidentRows * kFusedThreads / 64;
 
-// Form and threads of a single world's fused solve: a wavefront per chunk of a stage's constraints, up
-// to the form's limit; resident when all chunks fit.
-static FusedForm FusedPlan( const FusedArgs& a, int* threads )
+// Form and threads of a single world's fused solve: a wavefront per chunk of a stage's constraints and
+// at least a lane per kFusedBodyRegs bodies, up to the form's limit; resident when all chunks fit. Bodies
+// count too because a world in the air has hardly a chunk: 1,000 such bodies take 15 us per step this way
+// and 55 with a wavefront per chunk alone, 5,000 37 and 248; with two joined by a joint (general form)
+// 52 and 56, 88 and 115.
+static FusedForm FusedPlan( const FusedArgs& a, int chunks, int* threads )
 {
-	const int chunks = StageChunks( a.colorContactStart, a.colorJointStart, a.activeColorCount );
 	const FusedForm form = FusedIsGeneral( a ) ? kFusedGeneral : chunks <= kFusedResidentChunks ? kFusedResident : kFusedStreamed;
 	const int most = form == kFusedGeneral ? kFusedGeneralThreads : kFusedThreads;
 	*threads = 64;
-	while ( *threads < most && *threads < 64 * chunks )
+	while ( *threads < most && ( *threads < 64 * chunks || *threads * kFusedBodyRegs < a.bodyCount ) )
 	{
 		*threads *= 2;
 	}
@@ -2672,6 +2674,7 @@ __global__ __launch_bounds__( kThreads ) void SolveFlowKernel( FlowArgs a )
 struct FlowPlan
 {
 	void ( *kernel )( FlowArgs );
+	int rows;
 	int threads;
 };
 
@@ -2679,9 +2682,9 @@ static FlowPlan PlanFlow( int chunks, bool joints )
 {
 	if ( chunks <= 4 * 4 * kFlowGroups )
 	{
-		return joints ? FlowPlan{ SolveFlowKernel<4, 256, true>, 256 } : FlowPlan{ SolveFlowKernel<4, 256, false>, 256 };
+		return joints ? FlowPlan{ SolveFlowKernel<4, 256, true>, 4, 256 } : FlowPlan{ SolveFlowKernel<4, 256, false>, 4, 256 };
 	}
-	return joints ? FlowPlan{ SolveFlowKernel<2, 512, true>, 512 } : FlowPlan{ SolveFlowKernel<2, 512, false>, 512 };
+	return joints ? FlowPlan{ SolveFlowKernel<2, 512, true>, 2, 512 } : FlowPlan{ SolveFlowKernel<2, 512, false>, 2, 512 };
 }
 
 struct StoreArgs
@@ -4221,6 +4224,7 @@ struct DeviceWorld::Impl
 	SolverLists lists;
 	std::vector<int> slotStaging;
 	int solverPath = 0;
+	b2amd_SolverInfo lastSolver = {};
 	// step recording for the adjoint (null when not recording)
 	TapeStore* tape = nullptr;
 	int tapeIndex = 0;
@@ -5856,6 +5860,12 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 	{
 		solver = kSolverFused; // one workgroup per world; what does not fit is refused below
 	}
+	impl->lastSolver = {};
+	impl->lastSolver.chunks = StageChunks( L.colorContactStart, L.colorJointStart, L.activeColorCount );
+	if ( nb > 0 )
+	{
+		impl->lastSolver.path = solver == kSolverXcd ? b2amd_solverXcd : solver == kSolverFused ? b2amd_solverFused : b2amd_solverColorKernels;
+	}
 	if ( solver == kSolverXcd )
 	{
 		impl->EnsureFlow( nb, nc, ( 3 * kMaxColorSlots + 3 ) * (unsigned int)params.subStepCount );
@@ -6206,7 +6216,9 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 		impl->flowTag += ( 3 * kMaxColorSlots + 3 ) * (unsigned int)params.subStepCount;
 		double bytes = params.subStepCount * ( ( kBytesIntegrateVelocities + kBytesIntegratePositions ) * nb +
 											   ( kBytesWarmStart + kBytesSolve + kBytesRelax ) * nc + 3.0 * kBytesJoint * nj );
-		const FlowPlan plan = PlanFlow( StageChunks( xa.contactStart, xa.jointStart, xa.colors ), nj > 0 );
+		const FlowPlan plan = PlanFlow( impl->lastSolver.chunks, nj > 0 );
+		impl->lastSolver.form = plan.rows;
+		impl->lastSolver.threads = plan.threads;
 		impl->Launch( kkSolveXcd, bytes, [&]( hipEvent_t e0, hipEvent_t e1 ) {
 			hipExtLaunchKernelGGL( plan.kernel, dim3( kFlowGrid ), dim3( plan.threads ), 0, s, e0, e1, 0, xa );
 		} );
@@ -6251,7 +6263,9 @@ void DeviceWorld::SolveLaunch( const StepParams& params, bool anyRestitution, bo
 		else
 		{
 			int threads = 0;
-			const FusedForm form = FusedPlan( fa, &threads );
+			const FusedForm form = FusedPlan( fa, impl->lastSolver.chunks, &threads );
+			impl->lastSolver.form = form;
+			impl->lastSolver.threads = threads;
 			const auto kernel = form == kFusedGeneral ? SolveFusedKernel<kFusedGeneral>
 								: form == kFusedStreamed ? SolveFusedKernel<kFusedStreamed>
 														 : SolveFusedKernel<kFusedResident>;
@@ -6646,6 +6660,12 @@ void DeviceWorld::ResetKernelStats()
 		impl->statBytes[k] = 0.0;
 		impl->statLaunches[k] = 0;
 	}
+}
+
+b2amd_SolverInfo DeviceWorld::LastSolver() const
+{
+	JoinLaunch();
+	return impl->lastSolver;
 }
 
 void DeviceWorld::SetSolverPath( int path )

@@ -77,6 +77,22 @@ B2_API void b2amd_World_SetPairQuery( b2WorldId worldId, b2amd_PairQuery mode );
 /// pair update, 3 GPU speculative (run behind the previous step's solve).
 B2_API int b2amd_World_GetLastPairQuery( b2WorldId worldId );
 
+/// How the last step's substep loop ran.
+typedef struct b2amd_SolverInfo
+{
+	/// b2amd_solverColorKernels, b2amd_solverFused or b2amd_solverXcd; 0 before a step with awake bodies
+	int path;
+	/// fused: 0 general (joints, overflow constraints, restitution, warm start by body), 1 constraint
+	/// rows streamed, 2 rows resident in registers; XCD: rows a wavefront keeps in registers
+	int form;
+	/// workgroup size of the fused and XCD paths (0 in a batch, see b2amd_BatchStats)
+	int threads;
+	/// wavefronts' worth of constraints in a stage: 32 contacts or 64 joints of one color
+	int chunks;
+} b2amd_SolverInfo;
+
+B2_API b2amd_SolverInfo b2amd_World_GetLastSolver( b2WorldId worldId );
+
 /// Block until all GPU work issued by this library on the current device has completed
 /// (a device-wide synchronize; b2World_Step already returns with its own work complete).
 B2_API void b2amd_Synchronize( void );

@@ -103,3 +103,17 @@ def test_xcd_matches_color_kernels(gpu_scenes, kind, size, materials, steps):
     colored, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
     for k, (a, b) in enumerate(zip(xcd, colored)):
         assert a == b, f"step {k + 2}"
+
+
+@pytest.mark.parametrize("size", [100, 257, 1000, 5000])
+def test_bodies_in_the_air_have_lanes(gpu_scenes, size):
+    """Free fall: next to no constraints, but a lane for every two bodies up to the workgroup's limit."""
+    columns = 2 * int(size ** 0.5) + 4
+    h = gpu_scenes.create(box2d_amd.SCENE_RAIN, (size, columns, 0, 5), (1.5 * columns,))
+    try:
+        gpu_scenes.step(h, 5)
+        info = box2d_amd.last_solver(gpu_scenes.world_id(h))
+        assert info.path == box2d_amd.SOLVER_FUSED and info.chunks <= 2
+        assert 2 * info.threads >= min(size, 2048), info.threads
+    finally:
+        gpu_scenes.destroy(h)
