@@ -2283,6 +2283,7 @@ struct FlowPair
 			bodies[index].w = b.w;
 		}
 	}
+	static constexpr bool kJointBodiesLoaded = false;
 	B2G_DEVI static int JointA( const JointSim* )
 	{
 		return 0;

@@ -29,7 +29,7 @@ constexpr float kLengthUnitsPerMeter = 1.0f;
 struct RevoluteRow
 {
 	int type;
-	int bodyA, bodyB; // in the solver's body view
+	int bodyA, bodyB; // in the solver's body view; loaded, or the same for every joint
 	float mA, mB, iA, iB;
 	Softness softness;
 	b2Vec2 impulse;
@@ -37,11 +37,18 @@ struct RevoluteRow
 	b2Vec2 deltaCenter;
 	int spring, motor, limit;
 
-	// All loads have arrived after this.
+	// All loads have arrived after this. Indices that are constants of the view stay so: through the asm
+	// the compiler would lose them, and with them the registers of a view that they index (the XCD
+	// solver's two bodies of a joint went to 144 bytes of scratch and 16 KB of LDS).
+	template <typename Bodies>
 	B2G_DEVI void Await()
 	{
-		asm volatile( "" : "+v"( type ), "+v"( bodyA ), "+v"( bodyB ), "+v"( mA ), "+v"( mB ), "+v"( iA ), "+v"( iB ),
-					  "+v"( softness.biasRate ), "+v"( softness.massScale ), "+v"( softness.impulseScale ) );
+		asm volatile( "" : "+v"( type ), "+v"( mA ), "+v"( mB ), "+v"( iA ), "+v"( iB ), "+v"( softness.biasRate ),
+					  "+v"( softness.massScale ), "+v"( softness.impulseScale ) );
+		if constexpr ( Bodies::kJointBodiesLoaded )
+		{
+			asm volatile( "" : "+v"( bodyA ), "+v"( bodyB ) );
+		}
 		asm volatile( "" : "+v"( impulse.x ), "+v"( impulse.y ), "+v"( frameA.p.x ), "+v"( frameA.p.y ), "+v"( frameA.q.c ),
 					  "+v"( frameA.q.s ), "+v"( frameB.p.x ), "+v"( frameB.p.y ), "+v"( frameB.q.c ), "+v"( frameB.q.s ) );
 		asm volatile( "" : "+v"( deltaCenter.x ), "+v"( deltaCenter.y ), "+v"( spring ), "+v"( motor ), "+v"( limit ) );
@@ -66,7 +73,7 @@ B2G_DEVI RevoluteRow LoadRevoluteRow( const JointSim* j )
 					  j->enableSpring,
 					  j->enableMotor,
 					  j->enableLimit };
-	r.Await();
+	r.template Await<Bodies>();
 	return r;
 }
 

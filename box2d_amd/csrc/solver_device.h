@@ -192,6 +192,7 @@ struct GlobalBodies
 		}
 	}
 
+	static constexpr bool kJointBodiesLoaded = true; // JointA, JointB come from the joint's record
 	B2G_DEVI static int JointA( const JointSim* j )
 	{
 		return j->indexA;
@@ -243,6 +244,7 @@ struct LdsBodies
 		}
 	}
 
+	static constexpr bool kJointBodiesLoaded = true; // JointA, JointB come from the joint's record
 	B2G_DEVI static int JointA( const JointSim* j )
 	{
 		return j->slotA;
@@ -299,6 +301,7 @@ struct PackedBodies
 		}
 	}
 
+	static constexpr bool kJointBodiesLoaded = true; // JointA, JointB come from the joint's record
 	B2G_DEVI static int JointA( const JointSim* j )
 	{
 		return j->slotA;
