@@ -5763,26 +5763,34 @@ enum SolverKind
 	kSolverXcd,
 };
 
+// Constraint chunks up to which Auto prefers the fused solver for worlds with joints (see ChooseSolver).
+constexpr int kFusedJointChunks = 16;
+
 // path: b2amd_SolverPath. Auto takes the fused solver while a stage's chunks fit its wavefronts (the
 // resident form: measured 48 us per step for the 20-row pyramid, 55 for 24 rows, 64 for a 400-body
 // pile, against 65, 66 and 82 in the XCD solver), above that the XCD solver where it applies (26 rows
-// 66 against 120 us, 500 bodies 85 against 167, a 40x40 joint net 148 against 225; 100 rows 88 against
-// 279 in the color kernels, 20,000 bodies 288 against 689). Worlds it does not apply to (overflow
-// constraints, awake kinematic bodies) keep the fused solver up to kFusedMaxContacts contacts, where
-// its one launch beats the color kernels' about 70, and the color kernels beyond.
+// 66 against 120 us, 500 bodies 85 against 167; 100 rows 88 against 279 in the color kernels, 20,000
+// bodies 288 against 689). Worlds with joints have no resident form, and their general form pays a trip
+// to L2 per joint and color: the line lies lower for them. Fused against XCD solver: nets of 16, 20, 22,
+// 24 and 28 rows (10, 16, 18, 21 and 27 chunks) 95 and 113 us, 107 and 114, 113 and 113, 118 and 113, 135
+// and 113; piles of 40, 80, 100 and 300 bodies under a small net (11, 13, 16 and 27) 88 and 98, 94 and
+// 101, 129 and 96, 141 and 110. Worlds that the XCD solver does not apply to (overflow constraints, awake
+// kinematic bodies) keep the fused solver up to kFusedMaxContacts contacts, where its one launch beats the
+// color kernels' about 70, and the color kernels beyond.
 static SolverKind ChooseSolver( int path, const SolverLists& L, bool xcdUsable )
 {
 	const int nb = (int)L.awakeBodies.size();
 	const int nc = (int)L.constraintContacts.size();
 	const int overflow = L.overflowContactCount + L.overflowJointCount;
 	const bool colorsFit = L.activeColorCount <= kMaxColorSlots;
+	const int fusedChunks = L.jointList.empty() ? kFusedResidentChunks : kFusedJointChunks;
 	const bool fused = nb > 0 && nb <= kFusedBodyCapacity && colorsFit;
 	const bool xcd = xcdUsable && nb > 0 && nb <= kFlowMaxBodies && colorsFit && overflow == 0 && L.awakeKinematic == false;
 	switch ( path )
 	{
 		case 0:
-			return xcd && StageChunks( L.colorContactStart, L.colorJointStart, L.activeColorCount ) > kFusedResidentChunks ? kSolverXcd
-				   : fused && AutoFused( nc, overflow )																	   ? kSolverFused
+			return xcd && StageChunks( L.colorContactStart, L.colorJointStart, L.activeColorCount ) > fusedChunks ? kSolverXcd
+				   : fused && AutoFused( nc, overflow )																   ? kSolverFused
 																														   : kSolverColors;
 		case 2:
 			return fused ? kSolverFused : kSolverColors;

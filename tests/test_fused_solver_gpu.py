@@ -12,6 +12,7 @@ import pytest
 import box2d_amd
 from box2d_amd import WorldId
 from b2types import c_float
+from nets import add_net
 
 pytestmark = pytest.mark.gpu
 
@@ -115,5 +116,28 @@ def test_bodies_in_the_air_have_lanes(gpu_scenes, size):
         info = box2d_amd.last_solver(gpu_scenes.world_id(h))
         assert info.path == box2d_amd.SOLVER_FUSED and info.chunks <= 2
         assert 2 * info.threads >= min(size, 2048), info.threads
+    finally:
+        gpu_scenes.destroy(h)
+
+
+# (kind, size, joint net's rows), what Auto takes: worlds without joints fill the resident form's 32 chunks
+# first, those with joints go to the XCD solver above 16
+AUTO = [("pyramid", 24, 0, box2d_amd.SOLVER_FUSED), ("pyramid", 26, 0, box2d_amd.SOLVER_XCD),
+        ("pyramid", 1, 18, box2d_amd.SOLVER_FUSED), ("pyramid", 1, 26, box2d_amd.SOLVER_XCD),
+        ("pyramid", 14, 2, box2d_amd.SOLVER_XCD), ("pyramid", 8, 2, box2d_amd.SOLVER_FUSED)]
+
+
+@pytest.mark.parametrize("kind,size,net,path", AUTO)
+def test_auto_takes(gpu_scenes, kind, size, net, path):
+    h = gpu_scenes.pyramid(size, 100.0)
+    try:
+        world = gpu_scenes.world_id(h)
+        if net:
+            add_net(world, net)
+        gpu_scenes.step(h, 20)
+        info = box2d_amd.last_solver(world)
+        assert info.path == path, (info.path, info.chunks)
+        limit = 16 if net else 32
+        assert (info.chunks > limit) == (path == box2d_amd.SOLVER_XCD)
     finally:
         gpu_scenes.destroy(h)
