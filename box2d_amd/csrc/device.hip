@@ -5766,6 +5766,23 @@ enum SolverKind
 // Constraint chunks up to which Auto prefers the fused solver for worlds with joints (see ChooseSolver).
 constexpr int kFusedJointChunks = 16;
 
+// Whether a large world is still faster on the 32 CUs of one XCD than in the color kernels on all of
+// them. Those cost a launch per color and stage whatever the colors hold, so the line is one of
+// constraints per color, a joint counting as two and a half contacts; and beyond 32,768 bodies (the XCD
+// solver's body registers) each substep reads and writes the others. Color kernels against XCD solver:
+// pyramids (9 colors) of 48,510, 72,490, 86,280 and 134,850 contacts 285 and 173 us, 292 and 254, 297 and
+// 309, 314 and 505; nets (6 colors) of 16,020, 19,800, 28,560 and 124,500 joints 187 and 167, 186 and 185,
+// 193 and 241, 231 and 981; rain (19 colors) of 40,000, 50,000 and 100,000 bodies 769 and 532, 795 and 802,
+// 932 and 1,374.
+constexpr int kFlowContactsPerColor = 9000;
+constexpr int kFlowAutoBodies = 48 * 1024;
+
+static bool FlowPays( const SolverLists& L )
+{
+	const double constraints = (double)L.constraintContacts.size() + 2.5 * (double)L.jointList.size();
+	return (int)L.awakeBodies.size() <= kFlowAutoBodies && constraints <= (double)kFlowContactsPerColor * L.activeColorCount;
+}
+
 // path: b2amd_SolverPath. Auto takes the fused solver while a stage's chunks fit its wavefronts (the
 // resident form: measured 48 us per step for the 20-row pyramid, 55 for 24 rows, 64 for a 400-body
 // pile, against 65, 66 and 82 in the XCD solver), above that the XCD solver where it applies (26 rows
@@ -5774,7 +5791,7 @@ constexpr int kFusedJointChunks = 16;
 // to L2 per joint and color: the line lies lower for them. Fused against XCD solver: nets of 16, 20, 22,
 // 24 and 28 rows (10, 16, 18, 21 and 27 chunks) 95 and 113 us, 107 and 114, 113 and 113, 118 and 113, 135
 // and 113; piles of 40, 80, 100 and 300 bodies under a small net (11, 13, 16 and 27) 88 and 98, 94 and
-// 101, 129 and 96, 141 and 110. Worlds that the XCD solver does not apply to (overflow constraints, awake
+// 101, 129 and 96, 141 and 110. Very large worlds go back to the color kernels (FlowPays). Worlds that the XCD solver does not apply to (overflow constraints, awake
 // kinematic bodies) keep the fused solver up to kFusedMaxContacts contacts, where its one launch beats the
 // color kernels' about 70, and the color kernels beyond.
 static SolverKind ChooseSolver( int path, const SolverLists& L, bool xcdUsable )
@@ -5789,9 +5806,11 @@ static SolverKind ChooseSolver( int path, const SolverLists& L, bool xcdUsable )
 	switch ( path )
 	{
 		case 0:
-			return xcd && StageChunks( L.colorContactStart, L.colorJointStart, L.activeColorCount ) > fusedChunks ? kSolverXcd
-				   : fused && AutoFused( nc, overflow )																   ? kSolverFused
-																														   : kSolverColors;
+			if ( xcd && FlowPays( L ) && StageChunks( L.colorContactStart, L.colorJointStart, L.activeColorCount ) > fusedChunks )
+			{
+				return kSolverXcd;
+			}
+			return fused && AutoFused( nc, overflow ) ? kSolverFused : kSolverColors;
 		case 2:
 			return fused ? kSolverFused : kSolverColors;
 		case 3:

@@ -121,23 +121,25 @@ def test_bodies_in_the_air_have_lanes(gpu_scenes, size):
 
 
 # (kind, size, joint net's rows), what Auto takes: worlds without joints fill the resident form's 32 chunks
-# first, those with joints go to the XCD solver above 16
+# first, those with joints go to the XCD solver above 16; beyond 9,000 contacts a color, 3,600 joints a
+# color or 49,152 bodies the color kernels
 AUTO = [("pyramid", 24, 0, box2d_amd.SOLVER_FUSED), ("pyramid", 26, 0, box2d_amd.SOLVER_XCD),
         ("pyramid", 1, 18, box2d_amd.SOLVER_FUSED), ("pyramid", 1, 26, box2d_amd.SOLVER_XCD),
-        ("pyramid", 14, 2, box2d_amd.SOLVER_XCD), ("pyramid", 8, 2, box2d_amd.SOLVER_FUSED)]
+        ("pyramid", 14, 2, box2d_amd.SOLVER_XCD), ("pyramid", 8, 2, box2d_amd.SOLVER_FUSED),
+        ("pyramid", 225, 0, box2d_amd.SOLVER_XCD), ("pyramid", 250, 0, box2d_amd.SOLVER_COLOR_KERNELS),
+        ("pyramid", 1, 90, box2d_amd.SOLVER_XCD), ("pyramid", 1, 125, box2d_amd.SOLVER_COLOR_KERNELS)]
 
 
 @pytest.mark.parametrize("kind,size,net,path", AUTO)
 def test_auto_takes(gpu_scenes, kind, size, net, path):
-    h = gpu_scenes.pyramid(size, 100.0)
+    h = gpu_scenes.pyramid(size, 1000.0)
     try:
         world = gpu_scenes.world_id(h)
         if net:
             add_net(world, net)
-        gpu_scenes.step(h, 20)
+        gpu_scenes.step(h, 20 if max(size, net) < 90 else 4)
         info = box2d_amd.last_solver(world)
         assert info.path == path, (info.path, info.chunks)
-        limit = 16 if net else 32
-        assert (info.chunks > limit) == (path == box2d_amd.SOLVER_XCD)
+        assert (info.chunks > (16 if net else 32)) == (path != box2d_amd.SOLVER_FUSED)
     finally:
         gpu_scenes.destroy(h)
