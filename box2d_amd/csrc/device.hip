@@ -3891,8 +3891,8 @@ B2G_DEV void PackFinalizeBody( const PackFinalizeArgs& a )
 		a.mail[5] = 0;
 		if ( a.xcdSync != nullptr )
 		{
-			// a wait timed out, or no workgroup found itself on the solving XCD
-			a.mail[5] = a.xcdSync[2] != 0 || a.xcdSync[1] == 0 ? 1 : 0;
+			// 1 a wait timed out, 2 no workgroup found itself on the solving XCD
+			a.mail[5] = a.xcdSync[2] != 0 ? 1 : a.xcdSync[1] == 0 ? 2 : 0;
 			a.xcdSync[0] = 0;
 			a.xcdSync[1] = 0;
 			a.xcdSync[2] = 0;
@@ -4188,7 +4188,7 @@ struct DevArray
 	}
 };
 
-static bool XcdSolverUsable();
+static bool XcdSolverUsable( hipStream_t stream );
 static void AddReadbackUser();
 static void RemoveReadbackUser();
 
@@ -4369,7 +4369,7 @@ struct DeviceWorld::Impl
 	{
 		if ( xcdUsable < 0 )
 		{
-			xcdUsable = XcdSolverUsable() ? 1 : 0;
+			xcdUsable = XcdSolverUsable( stream ) ? 1 : 0;
 		}
 		return xcdUsable == 1;
 	}
@@ -5737,22 +5737,54 @@ static bool BatchWarmByBody( int bodyCount )
 	return BatchTuningFor( BatchBucketOf( bodyCount ) ).warmByBody != 0;
 }
 
+// Counts the workgroups of a launch like the XCD solver's that run on its XCD.
+__global__ void CountXcdGroupsKernel( int* count )
+{
+	if ( threadIdx.x == 0 && XccId() == 0 )
+	{
+		__hip_atomic_fetch_add( count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+	}
+}
+
+static_assert( kFlowGrid == kFlowGroups * kXcdCount, "one workgroup per CU" );
+
 // Whether the current device is one that the XCD solver is laid out for: an MI355X with all of its 8
-// XCDs of 32 CUs.
-static bool XcdSolverUsable()
+// XCDs of 32 CUs, whose launches place a workgroup in eight on the solving XCD. Where they do not (a CU
+// mask on the process) a step in that solver could only end in an error, so a launch finds out, once per
+// device and process.
+static bool XcdSolverUsable( hipStream_t stream )
 {
 	if ( getenv( "B2AMD_NO_XCD_SOLVER" ) != nullptr )
 	{
 		return false;
 	}
 	int device = 0;
-	hipDeviceProp_t prop;
-	if ( hipGetDevice( &device ) != hipSuccess || hipGetDeviceProperties( &prop, device ) != hipSuccess )
+	HIP_CHECK( hipGetDevice( &device ) );
+	static std::mutex mutex;
+	static std::map<int, bool> usable;
+	std::lock_guard<std::mutex> lock( mutex );
+	const auto known = usable.find( device );
+	if ( known != usable.end() )
 	{
-		(void)hipGetLastError();
-		return false;
+		return known->second;
 	}
-	return prop.multiProcessorCount == kFlowGrid && strncmp( prop.gcnArchName, "gfx950", 6 ) == 0;
+	hipDeviceProp_t prop;
+	HIP_CHECK( hipGetDeviceProperties( &prop, device ) );
+	bool ok = prop.multiProcessorCount == kFlowGrid && strncmp( prop.gcnArchName, "gfx950", 6 ) == 0;
+	if ( ok )
+	{
+		int groups = 0;
+		int* count = static_cast<int*>( s_devicePool.Alloc( sizeof( int ) ) );
+		HIP_CHECK( hipMemsetAsync( count, 0, sizeof( int ), stream ) );
+		CountXcdGroupsKernel<<<kFlowGrid, 64, 0, stream>>>( count );
+		HIP_CHECK( hipGetLastError() );
+		HIP_CHECK( hipMemcpyAsync( &groups, count, sizeof( int ), hipMemcpyDeviceToHost, stream ) );
+		HIP_CHECK( hipStreamSynchronize( stream ) );
+		s_devicePool.Free( count, sizeof( int ) );
+		ok = groups == kFlowGroups;
+	}
+	usable[device] = ok;
+	return ok;
 }
 
 // The solver of a world's step.
@@ -6589,7 +6621,8 @@ void DeviceWorld::SolveFinish( FinalizeResult* result )
 		}
 		if ( mail[5] != 0 )
 		{
-			Fatal( "XCD solver: a wait among its workgroups timed out (set B2AMD_NO_XCD_SOLVER to use the other solvers)" );
+			Fatal( "XCD solver: %s (set B2AMD_NO_XCD_SOLVER to use the other solvers)",
+				   mail[5] == 2 ? "no workgroup ran on the solving XCD" : "a wait among its workgroups timed out" );
 		}
 		result->enlargedBodies.assign( mail + kMailHeader, mail + kMailHeader + enlargedBodyCount );
 		result->enlargedShapes.assign( mail + pk.shapeOffset, mail + pk.shapeOffset + enlargedShapeCount );
