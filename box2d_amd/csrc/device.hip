@@ -4265,6 +4265,7 @@ struct DeviceWorld::Impl
 
 	// counters: [0..1] collide, [4..6] finalize
 	int* counters = nullptr;
+	bool countersCleared = false; // and the host knows
 	int* hostCounters = nullptr;
 
 	// Batched stepping: instead of launching, the phase functions record each kernel's
@@ -4602,10 +4603,9 @@ DeviceWorld::DeviceWorld()
 	impl = new Impl();
 	impl->stream = AcquireWorldStream( &impl->streamIndex );
 	impl->counters = static_cast<int*>( s_devicePool.Alloc( 16 * sizeof( int ) ) );
-	// zero once: from then on the pack kernels clear the counters after reading them. Waited for: a
-	// batch's kernels, on a stream of their own, may be the first to count.
+	// zero once: from then on the pack kernels clear the counters after reading them (a batch's kernels
+	// run on another stream: SetRecording waits for this)
 	HIP_CHECK( hipMemsetAsync( impl->counters, 0, 16 * sizeof( int ), impl->stream ) );
-	HIP_CHECK( hipStreamSynchronize( impl->stream ) );
 	impl->hostCounters = static_cast<int*>( s_pinnedPool.Alloc( 16 * sizeof( int ) ) );
 	for ( int i = 0; i < 4; ++i )
 	{
@@ -4698,6 +4698,7 @@ void DeviceWorld::UploadBodies( const World& world )
 	}
 	impl->bodyCount = n;
 	HIP_CHECK( hipStreamSynchronize( impl->stream ) );
+	impl->countersCleared = true;
 }
 
 // Readbacks between steps go through one pinned buffer that all worlds share: a kernel writes the
@@ -7392,6 +7393,11 @@ namespace b2g
 
 void DeviceWorld::SetRecording( bool flag )
 {
+	if ( impl->countersCleared == false )
+	{
+		HIP_CHECK( hipStreamSynchronize( impl->stream ) );
+		impl->countersCleared = true;
+	}
 	// Uploads and contact inits recorded but not taken by a batch run here, in order.
 	Impl::Record& r = impl->rec;
 	if ( r.uploads.empty() == false || r.init )
