@@ -1142,6 +1142,112 @@ B2G_DEVI void PrepareRev( const b2amd_TapeConstraint& r, RevConstraint& x )
 	adj[kaSep2] = sepb[1];
 }
 
+// Friction terms into the shapes, a shape's in constraint order. A constraint's sides hold its shapes
+// (FrictionSide) in c.slotA/slotB and their terms in adj[kaRA1X], adj[kaRA1Y]. Shapes of bodies that move
+// take theirs color by color with the pose terms (a body has one constraint of a color); those that several
+// constraints of a color share, the ground's above all, are left to one wavefront that walks the
+// constraints. In resident worlds each thread looks whether its constraint is the first of its shapes and
+// sums for those. Ten steps of two worlds of 1,541 bodies (4,565 contacts) take 69 ms with a loop over all
+// constraints for every shape and 13 this way, of 56 bodies and 5,000 static shapes 7.1 and 2.7.
+constexpr int kNoFriction = -1;
+
+B2G_DEVI int FrictionSide( int shapeId, int slot, const b2amd_TapeBody* bodies, bool colored )
+{
+	const bool own = colored && slot != kStaticSlot && ( bodies[slot - 1].flags & kDynamicFlag ) != 0;
+	return own ? shapeId : -2 - shapeId;
+}
+
+B2G_DEVI int FrictionShape( int side )
+{
+	return side <= -2 ? -2 - side : side;
+}
+
+B2G_DEV void SumFrictionResident( float* frictionGrad, const ConstraintSoA& c, const FieldTable& adj, int nc )
+{
+	const int tid = threadIdx.x;
+	if ( tid >= nc )
+	{
+		return;
+	}
+	const int shapeA = FrictionShape( c.slotA[tid] );
+	const int shapeB = FrictionShape( c.slotB[tid] );
+	bool firstA = shapeA != kNoFriction;
+	bool firstB = shapeB != kNoFriction;
+	float sumA = firstA ? frictionGrad[shapeA] : 0.0f;
+	float sumB = firstB ? frictionGrad[shapeB] : 0.0f;
+#pragma unroll 8
+	for ( int i = 0; i < nc; ++i )
+	{
+		const int a = FrictionShape( c.slotA[i] );
+		const int b = FrictionShape( c.slotB[i] );
+		const float ta = adj[kaRA1X][i];
+		const float tb = adj[kaRA1Y][i];
+		firstA = firstA && ( i >= tid || ( a != shapeA && b != shapeA ) );
+		firstB = firstB && ( i >= tid || ( a != shapeB && b != shapeB ) );
+		sumA = a == shapeA ? sumA + ta : b == shapeA ? sumA + tb : sumA;
+		sumB = a == shapeB ? sumB + ta : b == shapeB ? sumB + tb : sumB;
+	}
+	if ( firstA )
+	{
+		frictionGrad[shapeA] = sumA;
+	}
+	if ( firstB )
+	{
+		frictionGrad[shapeB] = sumB;
+	}
+}
+
+// The sides that are not a moving body's, by one wavefront. The sum of the shape at hand is lane 0's.
+B2G_DEV void SumFrictionOrdered( float* frictionGrad, const ConstraintSoA& c, const FieldTable& adj, int nc )
+{
+	const int lane = threadIdx.x;
+	int shape = kNoFriction;
+	float sum = 0.0f;
+	auto add = [&]( int side, float term ) {
+		const int next = -2 - side;
+		if ( next != shape )
+		{
+			if ( lane == 0 )
+			{
+				if ( shape != kNoFriction )
+				{
+					frictionGrad[shape] = sum;
+				}
+				sum = frictionGrad[next];
+			}
+			shape = next;
+		}
+		sum += term;
+	};
+	for ( int base = 0; base < nc; base += 64 )
+	{
+		const int i = b2MinInt( base + lane, nc - 1 );
+		const bool in = base + lane < nc;
+		const int sideA = in ? c.slotA[i] : kNoFriction;
+		const int sideB = in ? c.slotB[i] : kNoFriction;
+		const int termA = __float_as_int( adj[kaRA1X][i] );
+		const int termB = __float_as_int( adj[kaRA1Y][i] );
+		const unsigned long long left = __ballot( sideA <= -2 );
+		const unsigned long long right = __ballot( sideB <= -2 );
+		for ( unsigned long long any = left | right; any != 0; any &= any - 1 )
+		{
+			const int k = __ffsll( any ) - 1;
+			if ( left >> k & 1 )
+			{
+				add( __builtin_amdgcn_readlane( sideA, k ), __int_as_float( __builtin_amdgcn_readlane( termA, k ) ) );
+			}
+			if ( right >> k & 1 )
+			{
+				add( __builtin_amdgcn_readlane( sideB, k ), __int_as_float( __builtin_amdgcn_readlane( termB, k ) ) );
+			}
+		}
+	}
+	if ( lane == 0 && shape != kNoFriction )
+	{
+		frictionGrad[shape] = sum;
+	}
+}
+
 template <bool kResident>
 B2G_DEV void AdjointWorld( const AdjointWorldArgs& W, char* lds, int* s_unsupported, int* s_mismatch )
 {
@@ -1647,6 +1753,7 @@ B2G_DEV void AdjointWorld( const AdjointWorldArgs& W, char* lds, int* s_unsuppor
 		}
 
 		// ---- warm-start sources, preparation, manifold and friction terms ----
+		const int coloredEnd = colorStart( colors );
 		PoseTerms terms;
 		for ( int i = tid; i < nc; i += threads )
 		{
@@ -1709,8 +1816,8 @@ B2G_DEV void AdjointWorld( const AdjointWorldArgs& W, char* lds, int* s_unsuppor
 			float fB = W.shapes[r.shapeIdB].friction;
 			adj[kaRA1X][i] = friction ? fb * 0.5f * fB / fr : 0.0f;
 			adj[kaRA1Y][i] = friction ? fb * 0.5f * fA / fr : 0.0f;
-			c.slotA[i] = friction ? r.shapeIdA : -1;
-			c.slotB[i] = friction ? r.shapeIdB : -1;
+			c.slotA[i] = friction ? FrictionSide( r.shapeIdA, r.slotA, bodies, i < coloredEnd ) : kNoFriction;
+			c.slotB[i] = friction ? FrictionSide( r.shapeIdB, r.slotB, bodies, i < coloredEnd ) : kNoFriction;
 			if ( kResident )
 			{
 				terms = g;
@@ -1766,27 +1873,26 @@ B2G_DEV void AdjointWorld( const AdjointWorldArgs& W, char* lds, int* s_unsuppor
 						g.b[q] = adj[kaNX + 4 + q][i];
 					}
 					add( g, c.bodyA[i], c.bodyB[i] );
+					if ( c.slotA[i] >= 0 )
+					{
+						W.frictionGrad[c.slotA[i]] += adj[kaRA1X][i];
+					}
+					if ( c.slotB[i] >= 0 )
+					{
+						W.frictionGrad[c.slotB[i]] += adj[kaRA1Y][i];
+					}
 				}
 			}
 			sync();
 		}
 
-		// friction terms into the shapes, a shape's in constraint order
-		for ( int shape = tid; shape < W.shapeCap; shape += threads )
+		if ( kResident )
 		{
-			float sum = W.frictionGrad[shape];
-			for ( int i = 0; i < nc; ++i )
-			{
-				if ( c.slotA[i] == shape )
-				{
-					sum += adj[kaRA1X][i];
-				}
-				if ( c.slotB[i] == shape )
-				{
-					sum += adj[kaRA1Y][i];
-				}
-			}
-			W.frictionGrad[shape] = sum;
+			SumFrictionResident( W.frictionGrad, c, adj, nc );
+		}
+		else if ( tid < 64 )
+		{
+			SumFrictionOrdered( W.frictionGrad, c, adj, nc );
 		}
 		__syncthreads();
 	}

@@ -1,4 +1,5 @@
-"""A hanging net of balls on revolute joints, made through the public API: worlds with many joints."""
+"""Bodies made through the public API: hanging nets of balls on revolute joints (worlds with many joints),
+rows of static circles."""
 
 import ctypes
 
@@ -49,6 +50,14 @@ def add_body(world, kind, x, y, vx=0.0):
     body = _function("b2DefaultBodyDef", BodyDef)()
     body.type, body.position, body.linearVelocity = kind, Vec2(x, y), Vec2(vx, 0.0)
     return _function("b2CreateBody", Id, WorldId, ctypes.POINTER(BodyDef))(world, ctypes.byref(body))
+
+
+def add_circles(world, count, x):
+    """Static circles of radius 0.1 in a row from x on, 50 m up."""
+    shape = _function("b2DefaultShapeDef", ShapeDef)()
+    make_shape = _function("b2CreateCircleShape", Id, Id, ctypes.POINTER(ShapeDef), ctypes.POINTER(Circle))
+    for i in range(count):
+        make_shape(add_body(world, 0, x + 0.5 * i, 50.0), ctypes.byref(shape), ctypes.byref(Circle(Vec2(0.0, 0.0), 0.1)))
 
 
 def add_net(world, rows, spring=False):

@@ -7,6 +7,7 @@ import pytest
 
 from adjoint_ref import WorldRecord
 from earlier_work import EarlierWork
+from nets import add_circles
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,45 @@ def test_final_gradient_written_by_earlier_work(blocking):
         assert got.tobytes() == want.tobytes()
     finally:
         pw.destroy()
+
+
+@pytest.mark.parametrize("rows", [1, 5, 14, 17])
+def test_friction_gradients_of_all_shapes(rows):
+    """The ground's sum, which many constraints of a color share, and the boxes'."""
+    from box2d_amd.adjoint import BODY_STATE, PushWorlds
+
+    pw = PushWorlds(np.array([[5.5, 0.2, 0.4, 0.5]]), rows=rows)
+    try:
+        tape = pw.record(10)
+        final = tape.final_states()
+        target, pusher = int(pw.body_ids[0][0]), int(pw.body_ids[0][-1])
+        goal = np.array([0.5, rows - 1.0])
+        fg = np.zeros((1, tape.body_stride), dtype=BODY_STATE)
+        fg[0]["center"][target] = 2.0 * (final[0]["center"][target] - goal)
+        _, fr, stats = tape.backward(fg)
+        assert stats.unsupported == 0 and stats.replayMismatches == 0
+        rec = WorldRecord.from_tape(tape, 0)
+        _, want = rec.push_gradients(rec.slot_of(pusher), pw.pusher_shape_ids()[0], rec.slot_of(target), goal)
+        want = np.asarray(want["grad_friction"])[:fr.shape[1]]
+        assert np.count_nonzero(want) > rows
+        assert np.linalg.norm(fr[0][:len(want)] - want) <= 1e-3 * np.linalg.norm(want)
+    finally:
+        pw.destroy()
+
+
+def test_shapes_without_contacts_cost_nothing():
+    """The backward kernel's time does not grow with the world's shapes, only with its contacts."""
+    from box2d_amd.adjoint import BODY_STATE, PushWorlds
+
+    def milliseconds(extra):
+        pw = PushWorlds(np.array([[5.0, 0.1, 0.3, 0.5]]), rows=10)
+        try:
+            add_circles(pw.ids[0], extra, 200.0)
+            tape = pw.record(10)
+            fg = np.zeros((1, tape.body_stride), dtype=BODY_STATE)
+            fg["center"] = 1.0
+            return min(tape.backward(fg)[2].backwardMs for _ in range(3))
+        finally:
+            pw.destroy()
+
+    assert milliseconds(5000) < 1.5 * milliseconds(0)
