@@ -119,6 +119,33 @@ def test_batch_bucket_overrides_match_single_worlds(gpu_scenes, threads, warm):
             gpu_scenes.destroy(h)
 
 
+@pytest.mark.parametrize("threads", [64, 512, 1024])
+@pytest.mark.parametrize("joints", [False, True])
+def test_batch_of_one_form_matches_single_worlds(gpu_scenes, threads, joints):
+    """A batch without a world of the general form (no joints; its kernel leaves that form out), and the
+    same worlds beside one with joints."""
+    import box2d_amd
+
+    lib = box2d_amd.library()
+    specs = [(8, 0, 1), (40, 1, 2), (300, 0, 3), (600, 1, 4), (1500, 0, 5)] + [(60, 2, 6)] * joints
+    for k in range(4):
+        assert lib.b2amd_SetBatchTuning(k, threads, 0) == 0
+    batch = [gpu_scenes.create(box2d_amd.SCENE_BATCH_WORLD, spec) for spec in specs]
+    single = [gpu_scenes.create(box2d_amd.SCENE_BATCH_WORLD, spec) for spec in specs]
+    ids = (box2d_amd.WorldId * len(batch))(*[gpu_scenes.world_id(h) for h in batch])
+    try:
+        for step in range(40):
+            box2d_amd.step_worlds(ids)
+            for i, (hb, hs) in enumerate(zip(batch, single)):
+                gpu_scenes.step(hs)
+                assert gpu_scenes.hash(hb) == gpu_scenes.hash(hs), (step, specs[i])
+    finally:
+        for k in range(4):
+            lib.b2amd_SetBatchTuning(k, 0, 0)
+        for h in batch + single:
+            gpu_scenes.destroy(h)
+
+
 def test_batch_with_worlds_beyond_the_persistent_solver(gpu_scenes, world_runs):
     """Two 100-row pyramids (5050 bodies each) and a 105-row pyramid (5565 awake bodies, more than
     the persistent solver's 5400 LDS slots) batched with small worlds: the large world's substep

@@ -54,3 +54,9 @@ def test_xcd_solver(kernels, name, scratch):
     found = [v for k, v in kernels.items() if name in k]
     assert len(found) == 1
     assert found[0][0] <= scratch and found[0][1] <= 64, found
+
+
+@pytest.mark.parametrize("threads", [512, 1024])
+def test_batch_solver_without_general_worlds(kernels, threads):
+    found = [v for k, v in kernels.items() if f"SolveFusedBatchKernelILi{threads}ELb0E" in k]
+    assert len(found) == 1 and found[0][0] == 0, found
