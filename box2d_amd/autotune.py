@@ -7,8 +7,10 @@ threads, warm start body by body or color by color -- it steps a fresh copy of t
 the median GPU time of the persistent launch over the timed steps. The fastest configuration per
 bucket is written as the table of csrc/batch_tuning.h (rebuild the library to use it), and every
 timing to a markdown report. At run time each world takes its bucket's warm-start form, and a
-batch's single launch takes the workgroup size of the bucket that holds the most of its worlds. The configuration never changes a result, only the
-time; the batch tests check that for every workgroup size and both warm-start forms.
+batch's single launch takes the workgroup size of the bucket that holds the most of its worlds, so a size
+that is the fastest for small worlds alone may be too small for the large ones beside them: time uneven
+batches too before a new table is taken. The configuration never changes a result, only the time; the batch
+tests check that for every workgroup size and both warm-start forms.
 
     python -m box2d_amd.autotune --header gpurun_out/batch_tuning.h --report gpurun_out/batch_autotune.md
 """
