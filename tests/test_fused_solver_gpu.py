@@ -1,8 +1,9 @@
 """The single-workgroup solver's forms (rows resident in registers, rows streamed, general) and the XCD
-solver's (rows resident, more chunks than registers, joints) against the color kernels, bit for bit
-after every step, at the sizes where a form's chunks change: one chunk per color, partial chunks, the
-last resident world and the first streamed one, several chunks of one color in a wavefront, bodies
-without constraints."""
+solver's (four or two rows resident and the rest streamed, joints of every type) against the color kernels,
+bit for bit after every step, at the sizes where a form's chunks change: one chunk per color, partial
+chunks, the last resident world and the first streamed one, several chunks of one color in a wavefront,
+bodies without constraints, more bodies than registers. Each case states the form it is there for, and what
+the library reports of every step must agree. Then what Auto takes on either side of its lines."""
 
 import ctypes
 
@@ -12,6 +13,7 @@ import pytest
 import box2d_amd
 from box2d_amd import WorldId
 from b2types import c_float
+from box2d_amd.scenes_api import SCENE_JOINT_ZOO
 from nets import add_net
 
 pytestmark = pytest.mark.gpu
@@ -53,55 +55,76 @@ def _run(scenes, make, path, steps, materials):
         scenes.step(h, 1)
         if materials is not None:
             _set_materials(lib, world, materials == "bouncy")
-        out = []
+        out, used = [], []
         for _ in range(steps):
             scenes.step(h, 1)
             out.append((scenes.transforms(h).tobytes(), scenes.velocities(h).tobytes()))
-        return out, scenes.counters(h)["awake_contacts"]
+            info = box2d_amd.last_solver(world)
+            used.append((info.path, info.form, info.threads, info.chunks))
+        counters = scenes.counters(h)
+        return out, used, counters["awake_contacts"] + counters["joints"]
     finally:
         scenes.destroy(h)
 
 
-CASES = [("pyramid", rows, None, 40) for rows in (1, 2, 7, 11, 16, 21, 22, 23, 24, 25, 40)]
-CASES += [("pile", n, m, 150) for n in (1, 3, 33, 130) for m in (None, "rolling", "bouncy")]
-CASES += [("pile", 600, "rolling", 200), ("chains", 8, None, 40), ("chains", 160, None, 40), ("chains", 2600, None, 10)]
+GENERAL, STREAMED, RESIDENT = 0, 1, 2
+
+# (kind, size, materials, steps), the form that the last step takes
+CASES = [("pyramid", rows, None, 40, RESIDENT) for rows in (1, 2, 7, 11, 16, 21, 22, 23, 24, 25)]
+CASES += [("pyramid", rows, None, 40, STREAMED) for rows in (26, 40)]
+CASES += [("pile", n, m, 150, RESIDENT) for n in (1, 3, 33, 130) for m in (None, "rolling")]
+CASES += [("pile", n, "bouncy", 150, GENERAL) for n in (1, 3, 33, 130)]
+CASES += [("pile", 600, "rolling", 200, STREAMED)]
+CASES += [("chains", n, None, 40, GENERAL) for n in (8, 160)]
+CASES += [("net", rows, None, 20, GENERAL) for rows in (2, 12, 40)]
+CASES += [("zoo", 0, None, 60, GENERAL), ("hinges", 0, None, 100, GENERAL)]
 
 
-@pytest.mark.parametrize("kind,size,materials,steps", CASES)
-def test_fused_matches_color_kernels(gpu_scenes, kind, size, materials, steps):
-    def make():
-        if kind == "pyramid":
-            return gpu_scenes.pyramid(size)
-        if kind == "pile":
-            return gpu_scenes.create(box2d_amd.SCENE_MIXED_PILE, (size, 0, 77))
-        return gpu_scenes.create(box2d_amd.SCENE_BATCH_WORLD, (size, 2, 5))
+def _make(scenes, kind, size):
+    if kind == "pyramid":
+        return scenes.pyramid(size, 100.0)
+    if kind == "pile":
+        return scenes.create(box2d_amd.SCENE_MIXED_PILE, (size, 0, 77))
+    if kind == "zoo":
+        return scenes.create(SCENE_JOINT_ZOO, (0,))
+    if kind == "hinges":
+        return scenes.create(box2d_amd.SCENE_FALLING_HINGES)
+    if kind == "rain":
+        # spaced so that only a few neighbours touch: most bodies have no constraint; more bodies than the
+        # wavefronts keep in registers (16,384 with four rows, 32,768 with two)
+        return scenes.create(box2d_amd.SCENE_RAIN, (size, 170, 0, 9), (136.0,))
+    if kind == "net":
+        h = scenes.create(box2d_amd.SCENE_HELLO)
+        add_net(scenes.world_id(h), size, spring=size == 12)
+        return h
+    return scenes.create(box2d_amd.SCENE_BATCH_WORLD, (size, 2, 5))
 
-    fused, contacts = _run(gpu_scenes, make, box2d_amd.SOLVER_FUSED, steps, materials)
-    colored, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
-    assert kind == "chains" or contacts > 0
+
+@pytest.mark.parametrize("kind,size,materials,steps,form", CASES)
+def test_fused_matches_color_kernels(gpu_scenes, kind, size, materials, steps, form):
+    fused, used, constraints = _run(gpu_scenes, lambda: _make(gpu_scenes, kind, size), box2d_amd.SOLVER_FUSED, steps, materials)
+    colored, reference, _ = _run(gpu_scenes, lambda: _make(gpu_scenes, kind, size), box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
+    assert constraints > 0
+    assert {u[0] for u in used} == {box2d_amd.SOLVER_FUSED} and {u[0] for u in reference} == {box2d_amd.SOLVER_COLOR_KERNELS}
+    assert used[-1][1] == form, used[-1]
     for k, (a, b) in enumerate(zip(fused, colored)):
         assert a == b, f"step {k + 2}"
 
 
-XCD_CASES = [("pyramid", rows, None, 20) for rows in (1, 2, 7, 25, 60)] + [("pyramid", 112, None, 6)]
-XCD_CASES += [("pile", n, m, 120) for n in (1, 65, 600) for m in ("rolling", "bouncy")]
-XCD_CASES += [("chains", 160, None, 40), ("rain", 17000, None, 3)]
+# ..., rows that a wavefront keeps in registers: 4 up to 512 chunks, else 2
+XCD_CASES = [("pyramid", rows, None, 20, 4) for rows in (1, 2, 7, 25, 60)] + [("pyramid", 112, None, 6, 2)]
+XCD_CASES += [("pile", n, m, 120, 4) for n in (1, 65, 600) for m in ("rolling", "bouncy")]
+XCD_CASES += [("chains", 160, None, 40, 4), ("rain", 17000, None, 3, 4), ("rain", 34000, None, 2, 2), ("zoo", 0, None, 60, 4), ("hinges", 0, None, 100, 4)]
+XCD_CASES += [("net", rows, None, 10, 4) for rows in (2, 12, 70)] + [("net", 140, None, 4, 2)]
 
 
-@pytest.mark.parametrize("kind,size,materials,steps", XCD_CASES)
-def test_xcd_matches_color_kernels(gpu_scenes, kind, size, materials, steps):
-    def make():
-        if kind == "pyramid":
-            return gpu_scenes.pyramid(size, 100.0)
-        if kind == "rain":
-            # spaced so that only a few neighbours touch: most bodies have no constraint
-            return gpu_scenes.create(box2d_amd.SCENE_RAIN, (size, 170, 0, 9), (136.0,))
-        if kind == "pile":
-            return gpu_scenes.create(box2d_amd.SCENE_MIXED_PILE, (size, 0, 78))
-        return gpu_scenes.create(box2d_amd.SCENE_BATCH_WORLD, (size, 2, 6))
-
-    xcd, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_XCD, steps, materials)
-    colored, _ = _run(gpu_scenes, make, box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
+@pytest.mark.parametrize("kind,size,materials,steps,rows", XCD_CASES)
+def test_xcd_matches_color_kernels(gpu_scenes, kind, size, materials, steps, rows):
+    xcd, used, constraints = _run(gpu_scenes, lambda: _make(gpu_scenes, kind, size), box2d_amd.SOLVER_XCD, steps, materials)
+    colored, reference, _ = _run(gpu_scenes, lambda: _make(gpu_scenes, kind, size), box2d_amd.SOLVER_COLOR_KERNELS, steps, materials)
+    assert constraints > 0
+    assert {u[0] for u in used} == {box2d_amd.SOLVER_XCD} and {u[0] for u in reference} == {box2d_amd.SOLVER_COLOR_KERNELS}
+    assert used[-1][1] == rows, used[-1]
     for k, (a, b) in enumerate(zip(xcd, colored)):
         assert a == b, f"step {k + 2}"
 
