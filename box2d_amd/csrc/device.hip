@@ -4491,8 +4491,9 @@ struct DeviceWorld::Impl
 		cap = std::max<size_t>( cap, 64 );
 		if ( cfields.ptr != nullptr )
 		{
-			// another world may take the blocks at once
-			HIP_CHECK( hipDeviceSynchronize() );
+			// another world may take the blocks at once; only kernels on the world's own stream, and a
+			// batch's, which the batch has waited for, use them
+			HIP_CHECK( hipStreamSynchronize( stream ) );
 		}
 		cfields.Free();
 		cints.Free();
