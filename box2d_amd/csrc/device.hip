@@ -6999,9 +6999,9 @@ static void RunGeometryInDeviceMemory( const GeometryArray ( &arrays )[kArrays],
 	HIP_CHECK( hipFree( base ) );
 }
 
-// Run launch( arrays in the slot, records, stream ) over the records, a slot's worth at a time, after
-// the work that the default stream waits for (see AwaitDefaultStream); more than pinnedBytes of records
-// through device memory instead. Calls take turns.
+// Run launch( arrays in the slot, records, stream ) over the records, a slot's worth at a time; more
+// than pinnedBytes of records through device memory instead. Calls take turns. The callers have waited
+// for the default stream.
 template <int kArrays, typename Launch>
 static void RunGeometry( const GeometryArray ( &arrays )[kArrays], int count, size_t pinnedBytes, Launch launch )
 {
@@ -7019,7 +7019,6 @@ static void RunGeometry( const GeometryArray ( &arrays )[kArrays], int count, si
 	const int quarter = std::max( ( count - 1 ) / kGeometrySlots + 1, (int)( kGeometryLeastBytes / pairBytes ) );
 	const int most = std::min( ( quarter + kGeometryLanes - 1 ) / kGeometryLanes, (int)( kGeometrySlotBytes / pairBytes ) / kGeometryLanes ) *
 					 kGeometryLanes;
-	AwaitDefaultStream();
 	std::lock_guard<std::mutex> lock( s_geometry.mutex );
 	if ( s_geometry.ptr == nullptr )
 	{
@@ -7093,6 +7092,7 @@ int TimeOfImpactBatch( const b2TOIInput* inputs, int count, b2TOIOutput* outputs
 	{
 		return 0;
 	}
+	AwaitDefaultStream();
 	const GeometryArray arrays[2] = { { inputs, nullptr, sizeof( b2TOIInput ) }, { nullptr, outputs, sizeof( b2TOIOutput ) } };
 	RunGeometry( arrays, count, kTimeOfImpactPinnedBytes, []( char** at, int n, hipStream_t stream ) {
 		TimeOfImpactBatchKernel<<<GeometryBlocks( n ), kGeometryLanes, 0, stream>>>(
@@ -7107,6 +7107,7 @@ int ShapeDistanceBatch( const b2DistanceInput* inputs, b2SimplexCache* caches, i
 	{
 		return 0;
 	}
+	AwaitDefaultStream();
 	const GeometryArray arrays[3] = { { inputs, nullptr, sizeof( b2DistanceInput ) },
 									  { caches, caches, sizeof( b2SimplexCache ) },
 									  { nullptr, outputs, sizeof( b2DistanceOutput ) } };
@@ -7236,6 +7237,7 @@ int CollideBatch( const b2amd_Shape* shapesA, const b2amd_Shape* shapesB, const 
 		return 0;
 	}
 
+	AwaitDefaultStream();
 	for ( int i = 0; i < count; ++i )
 	{
 		if ( CollidePairSupported( shapesA[i].type, shapesB[i].type ) == false )

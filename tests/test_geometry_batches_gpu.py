@@ -78,5 +78,5 @@ def test_inputs_written_by_earlier_work(blocking):
         index = np.arange(9000) % len(a)
         a, b, x = _take(Shape, a, index), _take(Shape, b, index), _take(Transform, x, index)
         out = (LocalManifold * len(index))()
-        assert lib.b2amd_CollideBatch(a, b, work.writes(x), len(index), out) == 0
+        assert lib.b2amd_CollideBatch(work.writes(a), work.writes(b), work.writes(x), len(index), out) == 0
         assert np.array_equal(manifold_array_words(out), want[index])
