@@ -38,8 +38,8 @@ B2_API void b2amd_World_ResetKernelStats( b2WorldId worldId );
 /// kernel per graph color and stage; the XCD path runs the whole substep loop in one launch on the
 /// 32 compute units of one XCD, each constraint waiting for its own two bodies (MI355X only; worlds
 /// without overflow constraints and awake kinematic bodies). Auto picks the fused path for small
-/// worlds, the XCD path for larger ones where it applies and, where it does not, the fused path up to
-/// 4096 contact constraints and the color kernels beyond. Results are bit-identical across paths;
+/// worlds, the XCD path for larger ones where it applies, up to the size where all XCDs together are
+/// faster, and else the fused path up to 4096 contact constraints and the color kernels beyond. Results are bit-identical across paths;
 /// the switch exists for testing and measurement. Fused falls back to color kernels for worlds
 /// beyond its LDS budget, XCD to color kernels where it does not apply.
 typedef enum b2amd_SolverPath
@@ -121,7 +121,8 @@ typedef struct b2amd_Shape
 /// transforms[i] is the pose of B in A's frame (as for the reference b2Collide* functions).
 /// Pairs must be in the reference's primary order (A's type >= B's type in
 /// circle < capsule < segment < polygon, with segment-vs-polygon taking the segment as A).
-/// Host arrays in, host array out; synchronous. Returns 0 on success, -1 for an unsupported pair.
+/// Host arrays in, host array out; synchronous. Arrays are read after earlier work on the default
+/// stream, and on streams that wait for it. Returns 0 on success, -1 for an unsupported pair.
 B2_API int b2amd_CollideBatch( const b2amd_Shape* shapesA, const b2amd_Shape* shapesB, const b2Transform* transforms, int count,
 							   b2LocalManifold* manifolds );
 
@@ -148,7 +149,7 @@ typedef struct b2amd_BatchStats
 {
 	/// GPU time of the substep-loop launch over all worlds, milliseconds (HIP events)
 	float solveKernelMs;
-	/// workgroup size the autotuner chose (256, 512 or 1024)
+	/// workgroup size of that launch (64 to 1024)
 	int solveThreads;
 	/// number of persistent workgroups launched
 	int solveGrid;
